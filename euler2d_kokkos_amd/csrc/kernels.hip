@@ -132,9 +132,10 @@ struct P64 {
   // The march's primitive conversion keeps the reciprocal of the density for
   // the trace's source terms and checks both with one wave-level test.
   static constexpr bool kSharedRecip = true;
+  template <bool BND>
   static __device__ __forceinline__ bool prim_shared(const KParams &kp, const Cell &c, Q4T<T> &q,
                                                      double &r, bool &rok) {
-    return prim_fp64_shared(kp.s, c.u[0], c.u[1], c.u[2], c.u[3], q, r, rok);
+    return prim_fp64_shared<BND>(kp.s, c.u[0], c.u[1], c.u[2], c.u[3], q, r, rok);
   }
   static __device__ __forceinline__ void prim_ieee(const KParams &kp, const Cell &c, Q4T<T> &q) {
     prim_no_c<double, false>(kp.s, c.u[0], c.u[1], c.u[2], c.u[3], q);
@@ -882,13 +883,14 @@ __global__ void fluxes_atomic_kernel(KParams kp, Grid Q, Grid U, double dtdx, do
 // after the step, and the CFL rate of every updated cell is folded into a
 // wave max for the next launch's dt.
 
-// Whole-wavefront lane shifts by one with DPP (GFX9 wave_shr:1 / wave_shl:1):
-// a full-rate VALU move instead of an LDS-routed permute.  Lane 0 (shift up)
-// and lane 63 (shift down) read zero (bound_ctrl); the march never uses the
-// results of those lanes: the x-face of lane 1, the slopes of lanes 0 and 63
-// and the x-face of lane 63 feed only halo lanes.
-constexpr int kDppWaveShr1 = 0x138;  // lane i reads lane i-1
-constexpr int kDppWaveShl1 = 0x130;  // lane i reads lane i+1
+// Whole-wavefront lane rotations by one with DPP (GFX9 wave_ror:1 / wave_rol:1):
+// a full-rate VALU move instead of an LDS-routed permute.  Lanes 0 and 63 read
+// each other's state; the march never uses the results of those lanes (the
+// x-face of lane 1, the slopes of lanes 0 and 63 and the x-face of lane 63 feed
+// only halo lanes), but they are states in range, so that those lanes fail no
+// wave-level check.
+constexpr int kDppWaveRor1 = 0x13c;  // lane i reads lane i-1, lane 0 lane 63
+constexpr int kDppWaveRol1 = 0x134;  // lane i reads lane i+1, lane 63 lane 0
 
 template <int CTRL>
 __device__ __forceinline__ float dpp_shift(float x) {
@@ -908,14 +910,14 @@ __device__ __forceinline__ double dpp_shift(double x) {
 template <class T>
 __device__ __forceinline__ Q4T<T> shfl_up1(const Q4T<T> &a) {
   Q4T<T> r;
-  for (int v = 0; v < 4; v++) r.v[v] = dpp_shift<kDppWaveShr1>(a.v[v]);
+  for (int v = 0; v < 4; v++) r.v[v] = dpp_shift<kDppWaveRor1>(a.v[v]);
   return r;
 }
 
 template <class T>
 __device__ __forceinline__ Q4T<T> shfl_dn1(const Q4T<T> &a) {
   Q4T<T> r;
-  for (int v = 0; v < 4; v++) r.v[v] = dpp_shift<kDppWaveShl1>(a.v[v]);
+  for (int v = 0; v < 4; v++) r.v[v] = dpp_shift<kDppWaveRol1>(a.v[v]);
   return r;
 }
 
@@ -945,6 +947,9 @@ struct MarchState {
   // can equal the IEEE ones (its density and reciprocal normal)
   double rm1;
   bool rokm1;
+  // bounded FP64 kinds, wave-uniform: rows r-1 and r-2 passed the conversion's
+  // check; a cell outside the bounded ranges was met (or dt / dx is)
+  bool ok1, ok2, slow;
 };
 
 // One iteration over loaded row r.  STAGES is a compile-time set, so the
@@ -980,13 +985,24 @@ __device__ __forceinline__ void march_row(const KParams &kp, const Grid &in, con
       if (flipy) P::negate(dst, IV);
     }
   }
+  constexpr bool kMinmod = (RS & (kMinmodPow2 | kSlopeMinmod)) != 0;
+  // bounded kind: FP64 HLL / HLLC with the short root's conditions
+  constexpr bool kBnd = P::kSharedRecip && (RS & kRiemannFloorSqrt) != 0;
   Q4T<T> q0;
   [[maybe_unused]] double r0 = 0.0;
   [[maybe_unused]] bool rok0 = false, qok = true;
   if constexpr (P::kSharedRecip) {
-    qok = P::prim_shared(kp, uc, q0, r0, rok0);
+    qok = P::template prim_shared<kBnd>(kp, uc, q0, r0, rok0);
     if constexpr ((STAGES & kSlopes) == 0) {
-      if (!wave_all(qok)) P::prim_ieee(kp, uc, q0);  // uniform
+      const bool all = wave_all(qok);
+      if (!all) {  // uniform
+        P::prim_ieee(kp, uc, q0);
+        if constexpr (kBnd) m.slow = m.slow || !wave_all(!out_of_bounds(q0));
+      }
+      if constexpr (kBnd) {
+        m.ok2 = m.ok1;
+        m.ok1 = all;
+      }
     }
   } else {
     P::prim(kp, uc, q0);
@@ -998,46 +1014,81 @@ __device__ __forceinline__ void march_row(const KParams &kp, const Grid &in, con
     const Q4T<T> qpx = shfl_dn1(m.qm1);
     const Q4T<T> qmx = shfl_up1(m.qm1);
     Q4T<T> dqX = {}, dqY = {};
-    if constexpr ((RS & (kMinmodPow2 | kSlopeMinmod)) != 0) {  // slope_type == 1: no branch,
-                                                                // no products by one
+    if constexpr (kMinmod) {  // slope_type == 1: no branch, no products by one
       slopes_xy<true>(s.slope_type, m.qm1, qpx, qmx, q0, m.qm2, dqX, dqY);
     } else if (s.slope_type != T(0.0)) {  // uniform: one scalar branch per row
       slopes_xy<false>(s.slope_type, m.qm1, qpx, qmx, q0, m.qm2, dqX, dqY);
     }
     SourcesT<T> src;
-    if constexpr (P::kSharedRecip) {
+    Q4T<T> fymin, fxmin, fxmax;
+    auto y_faces = [&](auto half) {
+      trace_face<decltype(half)::value>(s, m.qm1, dqY, src, dtdy, false, fymin);
+      trace_face<decltype(half)::value>(s, m.qm1, dqY, src, dtdy, true, fymax);
+    };
+    auto x_faces = [&](auto half) {
+      if constexpr ((STAGES & kXFace) != 0) {
+        trace_face<decltype(half)::value>(s, m.qm1, dqX, src, dtdx, false, fxmin);
+        trace_face<decltype(half)::value>(s, m.qm1, dqX, src, dtdx, true, fxmax);
+      }
+    };
+    if constexpr (kBnd) {
+      // One check for row r's conversion; a wavefront with any lane outside the
+      // ranges there or in the two rows before (whose values the slopes of row a
+      // read) redoes the conversion, the slopes, the source terms and the face
+      // states as the reference writes them.
+      src = trace_sources_shared<true>(s, m.qm1, dqX, dqY, m.rm1, true, qok);
+      y_faces(std::true_type{});
+      x_faces(std::true_type{});
+      const bool all = wave_all(qok);
+      if (!(all && m.ok1 && m.ok2) || m.slow) {  // uniform
+        if (!all) P::prim_ieee(kp, uc, q0);
+        m.slow = m.slow || !wave_all(!out_of_bounds(q0));
+        if (s.slope_type != T(0.0))
+          slopes_xy<false>(s.slope_type, m.qm1, qpx, qmx, q0, m.qm2, dqX, dqY);
+        src = trace_sources(s, m.qm1, dqX, dqY);
+        y_faces(std::false_type{});
+        x_faces(std::false_type{});
+      }
+      m.ok2 = m.ok1;
+      m.ok1 = all;
+    } else if constexpr (P::kSharedRecip) {
       // one check for the quotients of row r's conversion and row a's source
       // terms; a wavefront with any lane outside the range redoes both, and
       // the y slopes that read row r, with the IEEE divisions
-      src = trace_sources_shared(s, m.qm1, dqX, dqY, m.rm1, m.rokm1, qok);
+      src = trace_sources_shared<false>(s, m.qm1, dqX, dqY, m.rm1, m.rokm1, qok);
       if (!wave_all(qok)) {  // uniform
         P::prim_ieee(kp, uc, q0);
-        if constexpr ((RS & (kMinmodPow2 | kSlopeMinmod)) != 0)
-          slopes_dir<true>(s.slope_type, m.qm1, q0, m.qm2, dqY);
-        else if (s.slope_type != T(0.0))
-          slopes_dir<false>(s.slope_type, m.qm1, q0, m.qm2, dqY);
+        if (s.slope_type != T(0.0)) slopes_dir<false>(s.slope_type, m.qm1, q0, m.qm2, dqY);
         src = trace_sources(s, m.qm1, dqX, dqY);
       }
     } else {
       src = trace_sources(s, m.qm1, dqX, dqY);
     }
-    Q4T<T> fymin;
-    trace_face(s, m.qm1, dqY, src, dtdy, false, fymin);
-    trace_face(s, m.qm1, dqY, src, dtdy, true, fymax);
-    if constexpr ((STAGES & kYFace) != 0) {
-      T f[4];
-      riemann<RS>(s, m.fymax_c, fymin, IV, IU, f);
-      for (int v = 0; v < 4; v++) fya.v[v] = f[v] * dtdy;
+    // the other kinds form the x faces after the y flux (fewer registers)
+    if constexpr (!kBnd) y_faces(std::false_type{});
+    bool fok = true;
+    T fy[4], fx[4];
+    if constexpr ((STAGES & kYFace) != 0) riemann<RS, kBnd>(s, m.fymax_c, fymin, IV, IU, fy, fok);
+    if constexpr (!kBnd) {
+      x_faces(std::false_type{});
     }
+    Q4T<T> ql;
     if constexpr ((STAGES & kXFace) != 0) {
-      Q4T<T> fxmin, fxmax;
-      trace_face(s, m.qm1, dqX, src, dtdx, false, fxmin);
-      trace_face(s, m.qm1, dqX, src, dtdx, true, fxmax);
-      const Q4T<T> ql = shfl_up1(fxmax);
-      T f[4];
-      riemann<RS>(s, ql, fxmin, IU, IV, f);
-      for (int v = 0; v < 4; v++) fxa.v[v] = f[v] * dtdx;
+      ql = shfl_up1(fxmax);
+      riemann<RS, kBnd>(s, ql, fxmin, IU, IV, fx, fok);
     }
+    if constexpr (kBnd && (STAGES & (kYFace | kXFace)) != 0) {
+      // the fluxes' quotients: one check for both faces, redone with the IEEE
+      // divisions in a wavefront with any lane outside
+      if (!wave_all(fok) || m.slow) {  // uniform
+        if constexpr ((STAGES & kYFace) != 0) riemann<RS>(s, m.fymax_c, fymin, IV, IU, fy);
+        if constexpr ((STAGES & kXFace) != 0) riemann<RS>(s, ql, fxmin, IU, IV, fx);
+      }
+    }
+    if constexpr ((STAGES & kYFace) != 0)
+      for (int v = 0; v < 4; v++) fya.v[v] = fy[v] * dtdy;
+    if constexpr ((STAGES & kXFace) != 0)
+      for (int v = 0; v < 4; v++) fxa.v[v] = fx[v] * dtdx;
     if constexpr ((STAGES & kUpdate) != 0) {
       const Q4T<T> fxr = shfl_dn1(m.fx_c);
       unew = P::update(m.ub, m.fx_c, fxr, m.fy_c, fya);
@@ -1160,6 +1211,8 @@ __device__ __forceinline__ typename P::T march(const KParams &kp, const Grid &in
   m.qm2 = m.qm1 = m.fymax_c = m.fx_c = m.fy_c = Q4T<T>{};
   m.rm1 = 0.0;
   m.rokm1 = false;
+  m.ok1 = m.ok2 = true;
+  m.slow = !wave_all((double)dtdx <= kBndDtd && (double)dtdy <= kBndDtd);
   m.wmax = T(0.0);
 
   const int r0 = j_base - 2;
@@ -1312,8 +1365,11 @@ __device__ __forceinline__ void fused_wave(const FusedMap &f, int wave, int &str
 
 // LOOP = false: explicit dt (HydroRun::godunov_unsplit); true: run-loop mode.
 // O32: 32-bit row offsets (every plane at most 4 GiB).
+// Two wavefronts per SIMD at least: the bounded FP64 kinds would otherwise take
+// 265 registers for the values their cold paths read, and run one.
 template <int RS, class P, bool LOOP, bool O32, int PD>
-__global__ __launch_bounds__(kBlock) void step_fused_kernel(KParams kp, Grid in, Grid out,
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(2)))
+void step_fused_kernel(KParams kp, Grid in, Grid out,
                                                             double dt_arg, StepCtl *ctl, int ph,
                                                             FusedMap fm) {
   using T = typename P::T;
@@ -1796,12 +1852,13 @@ KParams make_kparams(const e2d_params &p, int precision) {
   k.s.slope_type = p.slope_type;
   k.s.entho = 1.0 / (p.gamma0 - 1.0);
   k.s.smallc2 = p.smallc * p.smallc;
-  // the short square root for the wave speeds (arguments >= smallc^2) and
-  // the CFL rate (arguments >= about smallc^2 while d smallp is normal)
-  k.s.floor_sqrt =
-      k.s.smallc2 >= std::ldexp(1.0, -759) && p.smallr * p.smallp >= std::ldexp(1.0, -1000)
-          ? 1
-          : 0;
+  // the short square root for the wave speeds (arguments >= smallc^2) and the
+  // CFL rate, and the floors from which the bounded quotients' ranges follow
+  k.s.floor_sqrt = p.smallr >= std::ldexp(1.0, -60) && p.smallc >= std::ldexp(1.0, -60) &&
+                           p.smallr * p.smallp >= std::ldexp(1.0, -182) &&
+                           p.gamma0 <= 16.0 && k.s.entho <= std::ldexp(1.0, 20)
+                       ? 1
+                       : 0;
   k.s.riemann = p.honor_riemann ? p.riemannSolverType : 2;
   k.sf.gamma0 = (float)k.s.gamma0;
   k.sf.gamma6 = (float)k.s.gamma6;

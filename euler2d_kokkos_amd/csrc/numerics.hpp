@@ -45,8 +45,7 @@ struct Ops<double> {
 // x itself for +-0 and +inf.  For x in [2^-767, DBL_MAX] the scaling and the
 // special cases are identities, so the same core sequence, operation for
 // operation, gives the same bits; the host enables it only when smallc^2 (the
-// floor of every argument) is >= 2^-759.  A state with infinite pressure gets
-// NaN here where sqrt returns inf.
+// floor of every argument) is >= 2^-120.  +inf gives NaN where sqrt returns inf.
 __device__ __forceinline__ double sqrt_core(double x) {
   const double y = __builtin_amdgcn_rsq(x);
   double g = x * y;
@@ -83,19 +82,11 @@ struct SchemeT {
   T gamma0, gamma6, smallr, smallc, smallp, smallpp, slope_type, entho;
   T smallc2;    // smallc * smallc
   int riemann;  // 0 approx, 1 hll, 2 hllc (already resolved from honor_riemann)
-  int floor_sqrt;  // smallc2 >= 2^-759 and smallr*smallp >= 2^-1000: sound speeds take the short sqrt
+  // smallr and smallc >= 2^-60, smallr*smallp >= 2^-182, gamma0 <= 16, entho <= 2^20: the
+  // sound speeds take the short sqrt and the step's quotients the bounded forms
+  int floor_sqrt;
 };
 using Scheme = SchemeT<double>;
-
-// sqrt(x) for x >= s.smallc2 (the wave-speed estimates of the Riemann
-// solvers); FS selects the short sequence (FP64 only, when s.floor_sqrt)
-template <bool FS, class T>
-__device__ __forceinline__ T floored_sqrt(T x) {
-  if constexpr (FS)
-    return sqrt_core(x);
-  else
-    return Ops<T>::sqroot(x);
-}
 
 template <class T>
 struct Q4T {
@@ -106,18 +97,38 @@ using Q4 = Q4T<double>;
 // ------------------------------------------------ FP64 quotients sharing d
 // The compiler's IEEE FP64 division a / d is div_scale(d), rcp, two Newton
 // steps, m = a r, e = a - d m, q = m + e r (div_fmas), div_fixup.  For the
-// quotients of one cell by its density the reciprocal is formed once, by the
-// same operations, and each quotient takes the three steps after it.  The
-// scaling and fix-up steps act only where d or 1/d is not normal, where the
-// residual e is denormal (a below about 2^-969), or where q is not normal: the
-// class tests below catch each of these, and a wavefront with any such lane
-// takes the IEEE division for all of its lanes.  A zero quotient takes the
-// sign of m, as div_fixup gives it.  Same bits; 27 instead of 33 VALU
-// instructions for the three quotients of prim.  Each fallback is a branch
-// that splits the march's steady row, and a third branch per row measured
-// slower than no sharing at all; so quotients by one density that a row forms
-// later (the trace's source terms, the CFL rate's gamma p / d) join the check
-// of that density's conversion instead of adding one.
+// quotients by one d the reciprocal is formed once, by the same operations,
+// and each quotient takes the three steps after it.  The scaling and fix-up
+// steps act only where d or 1/d is not normal, where the residual e is
+// denormal (a below about 2^-969), or where q is not normal: class tests catch
+// each of these, and a wavefront with any such lane takes the IEEE division
+// for all of its lanes.  A zero quotient takes the sign of m, as div_fixup
+// gives it.  Same bits; 27 instead of 33 VALU instructions for the three
+// quotients of prim.  Each fallback is a branch that splits the march's steady
+// row; so quotients by one density that a row forms later (the trace's source
+// terms, the CFL rate's gamma p / d) join the check of that density's
+// conversion instead of adding one.
+//
+// Bounded kinds (BND).  Where the floors of the deck are not absurdly small
+// (SchemeT::floor_sqrt, decided on the host) most of those tests follow from
+// ranges that are cheap to check once per cell:
+//   d <= 2^40, p <= 2^90, (u^2 + v^2) / 2 <= 2^100, and the residuals of the
+//   quotients u, v and E / d zero or normal.
+// Then smallr >= 2^-60 <= d makes d and 1/d normal; a normal residual means a
+// numerator of at least 2^-970, so u, v and E / d are zero or at least 2^-1010,
+// and their differences zero or at least 2^-1062; p >= smallr smallp >= 2^-182
+// makes pressure differences zero or at least 2^-235.  With dt / dx <= 2^40
+// (checked per wavefront) the traced face states stay below 2^190 in density,
+// pressure and velocity, far from overflow in every product of the solvers.
+// A wavefront with a lane outside these ranges takes the IEEE divisions.
+//
+// The march is bound by VALU issue (4 cycles per FP64 instruction, 16 per rcp
+// or rsq), so these forms, one wave-speed root per face instead of two, the
+// minmod slope without its redundant third limit, one side's energy per HLLC
+// face and no branch between its two fluxes count directly: a steady HLLC row
+// went from 695 instructions (2900 issue cycles) to 590 (2420).  1024x1536
+// blast, 14-row tile: 50.3 -> 44.7 us a step; 8192x8192, 48 rows: HLLC 1874 -> 1579,
+// HLL 1701 -> 1510 us.
 
 __device__ __forceinline__ double recip_newton(double d) {
   const double r0 = __builtin_amdgcn_rcp(d);
@@ -127,6 +138,24 @@ __device__ __forceinline__ double recip_newton(double d) {
 
 constexpr int kClassNormal = (1 << 3) | (1 << 8);
 constexpr int kClassZeroOrNormal = kClassNormal | (1 << 5) | (1 << 6);
+
+constexpr double kBndDensity = 0x1p40, kBndPressure = 0x1p90, kBndKinetic = 0x1p100;
+constexpr double kBndDtd = 0x1p40;  // dt / dx, dt / dy
+
+// a / d from r = 1 / d where no step needs scaling and a is not -0
+__device__ __forceinline__ double quot_plain(double a, double d, double r) {
+  const double m = a * r;
+  return __builtin_fma(__builtin_fma(-d, m, a), r, m);
+}
+
+// the same with the residual's test: ok is cleared where it is denormal, or
+// where a step overflowed or met a NaN
+__device__ __forceinline__ double quot_resid(double a, double d, double r, bool &ok) {
+  const double m = a * r;
+  const double e = __builtin_fma(-d, m, a);
+  ok = ok && __builtin_amdgcn_class(e, kClassZeroOrNormal);
+  return __builtin_fma(e, r, m);
+}
 
 __device__ __forceinline__ double quot_shared(double a, double d, double r, bool &ok) {
   const double m = a * r;
@@ -142,9 +171,10 @@ __device__ __forceinline__ bool wave_all(bool ok) {
   return __builtin_amdgcn_ballot_w64(!ok) == 0;
 }
 
-// the rest of computePrimitives once the three quotients are formed
-__device__ __forceinline__ void prim_finish(const SchemeT<double> &s, double d, double ux,
-                                            double uy, double e1, Q4T<double> &q) {
+// the rest of computePrimitives once the three quotients are formed; returns
+// the specific kinetic energy
+__device__ __forceinline__ double prim_finish(const SchemeT<double> &s, double d, double ux,
+                                              double uy, double e1, Q4T<double> &q) {
   const double eken = 0.5 * (uy * uy + ux * ux);
   const double e = e1 - eken;
   const double p = fmax((s.gamma0 - 1.0) * d * e, d * s.smallp);
@@ -152,24 +182,43 @@ __device__ __forceinline__ void prim_finish(const SchemeT<double> &s, double d, 
   q.v[IP] = p;
   q.v[IU] = ux;
   q.v[IV] = uy;
+  return eken;
+}
+
+// the cell is outside the ranges of the bounded kinds (a NaN counts as outside)
+__device__ __forceinline__ bool out_of_bounds(const Q4T<double> &q) {
+  const double eken = 0.5 * (q.v[IV] * q.v[IV] + q.v[IU] * q.v[IU]);
+  return !(q.v[ID] <= kBndDensity && q.v[IP] <= kBndPressure && eken <= kBndKinetic);
 }
 
 // computePrimitives for FP64 with the three quotients formed from one
 // reciprocal and no fallback.  Returns whether this lane's quotients are the
-// IEEE ones; r is the reciprocal and rok whether other quotients by d formed
-// from it can be (d and r normal).
+// IEEE ones (BND: and the cell is in the bounded ranges); r is the reciprocal
+// and rok whether other quotients by d formed from it can be (d and r normal;
+// BND: part of the result instead).
+template <bool BND = false>
 __device__ __forceinline__ bool prim_fp64_shared(const SchemeT<double> &s, double u0, double u1,
                                                  double u2, double u3, Q4T<double> &q, double &r,
                                                  bool &rok) {
   const double d = fmax(u0, s.smallr);
   r = recip_newton(d);
-  rok = __builtin_amdgcn_class(d, kClassNormal) && __builtin_amdgcn_class(r, kClassNormal);
-  bool ok = rok;
-  const double ux = quot_shared(u2, d, r, ok);
-  const double uy = quot_shared(u3, d, r, ok);
-  const double e1 = quot_shared(u1, d, r, ok);
-  prim_finish(s, d, ux, uy, e1, q);
-  return ok;
+  if constexpr (BND) {
+    rok = true;
+    bool ok = d <= kBndDensity;
+    const double ux = __builtin_copysign(quot_resid(u2, d, r, ok), u2);  // d > 0
+    const double uy = __builtin_copysign(quot_resid(u3, d, r, ok), u3);
+    const double e1 = quot_resid(u1, d, r, ok);
+    const double eken = prim_finish(s, d, ux, uy, e1, q);
+    return ok && q.v[IP] <= kBndPressure && eken <= kBndKinetic;
+  } else {
+    rok = __builtin_amdgcn_class(d, kClassNormal) && __builtin_amdgcn_class(r, kClassNormal);
+    bool ok = rok;
+    const double ux = quot_shared(u2, d, r, ok);
+    const double uy = quot_shared(u3, d, r, ok);
+    const double e1 = quot_shared(u1, d, r, ok);
+    prim_finish(s, d, ux, uy, e1, q);
+    return ok;
+  }
 }
 
 // computePrimitives for FP64: the shared reciprocal, and the IEEE divisions
@@ -252,11 +301,10 @@ __device__ __forceinline__ T cfl_rate_q(const SchemeT<T> &s, const Q4T<T> &q, co
   return rx + ry;
 }
 
-// The rate's square root of gamma p / d.  p >= d smallp, and with smallc^2 >=
-// 2^-759 and smallr smallp >= 2^-1000 (the host's floor_sqrt condition, which
-// keeps d smallp normal for every d >= smallr) the argument is at least
-// smallc^2 (1 - 5u) > 2^-767, where the short sequence gives the IEEE bits;
-// +inf keeps sqrt's result, and NaN stays NaN.
+// The rate's square root of gamma p / d.  p >= d smallp, and under the host's
+// floor_sqrt condition (which keeps d smallp normal for every d >= smallr) the
+// argument is at least smallc^2 (1 - 5u) > 2^-121, where the short sequence gives
+// the IEEE bits; +inf keeps sqrt's result, and NaN stays NaN.
 template <bool FS>
 __device__ __forceinline__ double rate_sqrt(double x) {
   if constexpr (FS) {
@@ -274,14 +322,16 @@ __device__ __forceinline__ double rate_sqrt(double x) {
 // cfl_rate_q for FP64 from the conserved state: the quotient gamma p / d
 // shares the primitive conversion's reciprocal and its one wave-level check.
 // POW2: both cell sizes are known to be powers of two (no test per cell).
-template <bool FS, bool POW2 = false>
+template <bool FS, bool POW2 = false>  // FS: also the bounded kinds' conversion
 __device__ __forceinline__ double cfl_rate_fp64(const Scheme &s, double u0, double u1, double u2,
                                                 double u3, const RateT<double> &rt) {
   Q4 q;
   double r;
   bool rok;
-  bool ok = prim_fp64_shared(s, u0, u1, u2, u3, q, r, rok);
-  double x = quot_shared(s.gamma0 * q.v[IP], q.v[ID], r, rok);
+  bool ok = prim_fp64_shared<FS>(s, u0, u1, u2, u3, q, r, rok);
+  // bounded: smallp <= p / d <= 2^150, nothing to scale
+  double x = FS ? quot_plain(s.gamma0 * q.v[IP], q.v[ID], r)
+                : quot_shared(s.gamma0 * q.v[IP], q.v[ID], r, rok);
   if (!wave_all(ok && rok)) {  // uniform
     prim_no_c<double, false>(s, u0, u1, u2, u3, q);
     x = (s.gamma0 * q.v[IP]) / q.v[ID];
@@ -309,12 +359,30 @@ __device__ __forceinline__ double cfl_rate(const Scheme &s, double u0, double u1
   return cfl_rate_q(s, q, dx, dy);
 }
 
+// neg ? -z : z as one select on the high word (with the operand's negation)
+__device__ __forceinline__ double select_neg(bool neg, double z) {
+  const long long b = __double_as_longlong(z);
+  const float h = __int_as_float((int)(b >> 32));
+  const int hi = __float_as_int(neg ? -h : h);
+  return __longlong_as_double(((long long)hi << 32) | (unsigned int)b);
+}
+__device__ __forceinline__ float select_neg(bool neg, float z) { return neg ? -z : z; }
+
 // slope_unsplit_hydro_2d_scalar, HydroBaseFunctor.h:419-455 (one direction).
 // MINMOD: st == 1, whose products with the one-sided differences are exact
 // identities (every value, zeros, infinities and NaN included) and are left out.
 template <bool MINMOD = false, class T>
 __device__ __forceinline__ T limited_slope(T st, T q, T qplus, T qminus) {
   using O = Ops<T>;
+  if constexpr (MINMOD && sizeof(T) == sizeof(double)) {
+    // The sum of two one-sided differences of one sign is at least twice the
+    // smaller, after rounding too, so |dcen| never limits them; and dcen >= 0
+    // where qplus >= qminus, except that qminus - qplus = 2^-1074 halves to -0:
+    // callers keep to values whose differences are zero or larger than that.
+    const T dl = q - qminus, dr = qplus - q;
+    const T z = (dl * dr <= T(0.0)) ? T(0.0) : O::mn(O::ab(dl), O::ab(dr));
+    return select_neg(!(qplus >= qminus), z);
+  }
   const T dlft = MINMOD ? q - qminus : st * (q - qminus);
   const T drgt = MINMOD ? qplus - q : st * (qplus - q);
   const T dcen = T(0.5) * (qplus - qminus);
@@ -379,7 +447,9 @@ __device__ __forceinline__ SourcesT<T> trace_sources(const SchemeT<T> &s, const 
 // trace_sources for FP64 with the two pressure-slope quotients formed from the
 // reciprocal rinv of the density q.v[ID] that the primitive conversion made
 // (rok: d and rinv normal), with no fallback; ok is cleared in a lane whose
-// quotients may differ from the IEEE ones.
+// quotients may differ from the IEEE ones (BND: none does where the cells are in
+// the bounded ranges).
+template <bool BND>
 __device__ __forceinline__ Sources trace_sources_shared(const Scheme &s, const Q4 &q,
                                                         const Q4 &dqX, const Q4 &dqY, double rinv,
                                                         bool rok, bool &ok) {
@@ -389,61 +459,96 @@ __device__ __forceinline__ Sources trace_sources_shared(const Scheme &s, const Q
   const double divu = dqX.v[IU] + dqY.v[IV];
   o.sr0 = O::mad(-divu, r, O::mad(-v, dqY.v[ID], -u * dqX.v[ID]));
   o.sp0 = O::mad(-(divu * s.gamma0), p, O::mad(-v, dqY.v[IP], -u * dqX.v[IP]));
-  bool qok = rok;
-  const double qx = quot_shared(dqX.v[IP], r, rinv, qok);
-  const double qy = quot_shared(dqY.v[IP], r, rinv, qok);
-  ok = ok && qok;
+  double qx, qy;
+  if constexpr (BND) {
+    qx = __builtin_copysign(quot_plain(dqX.v[IP], r, rinv), dqX.v[IP]);
+    qy = __builtin_copysign(quot_plain(dqY.v[IP], r, rinv), dqY.v[IP]);
+  } else {
+    bool qok = rok;
+    qx = quot_shared(dqX.v[IP], r, rinv, qok);
+    qy = quot_shared(dqY.v[IP], r, rinv, qok);
+    ok = ok && qok;
+  }
   o.su0 = O::mad(-v, dqY.v[IU], -u * dqX.v[IU]) - qx;
   o.sv0 = O::mad(-v, dqY.v[IV], -u * dqX.v[IV]) - qy;
   return o;
 }
 
+__device__ __forceinline__ double fma_t(double a, double b, double c) {
+  return __builtin_fma(a, b, c);
+}
+__device__ __forceinline__ float fma_t(float a, float b, float c) {
+  return __builtin_fmaf(a, b, c);
+}
+
 // Face states of trace_unsplit_2d_along_dir, HydroBaseFunctor.h:251-289.
 // plus = false for the XMIN / YMIN faces, true for XMAX / YMAX; dq is the
 // slope along the face normal, dtd = dtdx or dtdy.
-template <class T>
+// HALF: the product of the slope by a half is exact (bounded kinds), so that it
+// may be fused with the sum.
+template <bool HALF = false, class T>
 __device__ __forceinline__ void trace_face(const SchemeT<T> &s, const Q4T<T> &q, const Q4T<T> &dq,
                                            const SourcesT<T> &src, T dtd, bool plus, Q4T<T> &f) {
   using O = Ops<T>;
   // (q +- h*dq) + (src*dtd)*h
   const T h = T(0.5), hs = plus ? h : -h;
-  f.v[ID] = O::mad(src.sr0 * dtd, h, O::mad(hs, dq.v[ID], q.v[ID]));
-  f.v[IP] = O::mad(src.sp0 * dtd, h, O::mad(hs, dq.v[IP], q.v[IP]));
-  f.v[IU] = O::mad(src.su0 * dtd, h, O::mad(hs, dq.v[IU], q.v[IU]));
-  f.v[IV] = O::mad(src.sv0 * dtd, h, O::mad(hs, dq.v[IV], q.v[IV]));
+  const T t[4] = {src.sr0, src.sp0, src.su0, src.sv0};
+  for (int v = 0; v < 4; v++) {
+    const T e = HALF ? fma_t(hs, dq.v[v], q.v[v]) : O::mad(hs, dq.v[v], q.v[v]);
+    f.v[v] = O::mad(t[v] * dtd, h, e);
+  }
   f.v[ID] = O::mx(s.smallr, f.v[ID]);
+}
+
+// Largest sound speed of the two states of a face, floored at smallc:
+// max(sqrt(max(gamma p / r, smallc^2))) over the two.  A correctly rounded
+// square root never decreases where its argument grows, so the root of the
+// larger argument is the larger root, bit for bit, and one root serves both
+// (the FP32 hardware root was checked to be monotone over every positive float).
+// FS: the short root, which gives NaN for +inf: its argument is capped at the
+// largest finite value.  BND: quotients of states in the bounded ranges.
+template <bool FS, bool BND, class T>
+__device__ __forceinline__ T wave_speed(const SchemeT<T> &s, T pl, T rl, T pr, T rr) {
+  using O = Ops<T>;
+  if constexpr (BND) {
+    const T xl = quot_plain(s.gamma0 * pl, rl, recip_newton(rl));
+    const T xr = quot_plain(s.gamma0 * pr, rr, recip_newton(rr));
+    return sqrt_core(O::mx(O::mx(xl, xr), s.smallc2));
+  } else {
+    const T a = O::mx(O::mx(O::div(s.gamma0 * pl, rl), O::div(s.gamma0 * pr, rr)), s.smallc2);
+    if constexpr (FS) return sqrt_core(O::mn(a, T(__DBL_MAX__)));
+    return O::sqroot(a);
+  }
 }
 
 // riemann_hllc, HydroBaseFunctor.h:704-809.  `ln`/`tn` are the indices of the
 // normal / transverse velocity in the Q4 (IU/IV for x faces, IV/IU for y faces,
 // which is the reference's swap before and after the call, :628-632).
 // The reference evaluates both star states and then picks one; here the side
-// (left if ustar > 0) is picked first and its star state evaluated once with
-// the same expressions, which gives identical bits for the state it keeps.
-template <bool FS = false, class T>
+// is picked first and its energy, star state and outer state are evaluated
+// once with the same expressions, which gives identical bits for the state
+// it keeps: the left side where ustar > 0 or SL > 0 (there the reference takes
+// the left state itself), the right one elsewhere.
+// BND: the two quotients by rcr + rcl share a reciprocal, as do the two by
+// Sk - ustar; ok is cleared in a lane where one of them may differ from the
+// IEEE quotient.  Of the bounded ranges' consequences these are left to test:
+// rcr + rcl and Sk - ustar away from zero, and the residuals of ustar and
+// etotstar, whose numerators may be tiny (those of ptotstar and rstar are
+// zero or at least 2^-410; an overflow anywhere makes the last residual NaN
+// or infinite).  No numerator is ever -0: each ends in a sum with +0 or with a
+// number that is not zero.
+template <bool FS = false, bool BND = false, class T>
 __device__ __forceinline__ void hllc(const SchemeT<T> &s, const Q4T<T> &ql, const Q4T<T> &qr,
-                                     int ln, int tn, T flux[4]) {
+                                     int ln, int tn, T flux[4], bool &ok) {
   using O = Ops<T>;
   const T h = T(0.5);
-  const T rl = O::mx(ql.v[ID], s.smallr);
+  // the reference floors the densities at smallr again; trace_face has done it
+  const T rl = ql.v[ID], rr = qr.v[ID];
   const T pl = O::mx(ql.v[IP], rl * s.smallp);
-  const T ul = ql.v[ln];
-  T ecinl = h * rl * ul * ul;
-  ecinl = O::mad(h * rl * ql.v[tn], ql.v[tn], ecinl);
-  const T etotl = O::mad(pl, s.entho, ecinl);
-  const T ptotl = pl;
-
-  const T rr = O::mx(qr.v[ID], s.smallr);
   const T pr = O::mx(qr.v[IP], rr * s.smallp);
-  const T ur = qr.v[ln];
-  T ecinr = h * rr * ur * ur;
-  ecinr = O::mad(h * rr * qr.v[tn], qr.v[tn], ecinr);
-  const T etotr = O::mad(pr, s.entho, ecinr);
-  const T ptotr = pr;
+  const T ul = ql.v[ln], ur = qr.v[ln];
 
-  const T cfastl = floored_sqrt<FS>(O::mx(O::div(s.gamma0 * pl, rl), s.smallc2));
-  const T cfastr = floored_sqrt<FS>(O::mx(O::div(s.gamma0 * pr, rr), s.smallc2));
-  const T cmax = O::mx(cfastl, cfastr);
+  const T cmax = wave_speed<FS, BND>(s, pl, rl, pr, rr);
   const T SL = O::mn(ul, ur) - cmax;
   const T SR = O::mx(ul, ur) + cmax;
 
@@ -451,27 +556,56 @@ __device__ __forceinline__ void hllc(const SchemeT<T> &s, const Q4T<T> &ql, cons
   const T rcr = rr * (SR - ur);
   // separate products: for mirrored states at a reflecting wall they cancel
   // exactly, so ustar and the wall's mass flux are exactly zero
-  const T ustar = O::div(rcr * ur + rcl * ul + (ptotl - ptotr), rcr + rcl);
+  const T un = rcr * ur + rcl * ul + (pl - pr);
   // the left/right-symmetric sum stays unfused, so that mirrored states give
   // mirrored fluxes in FP32 too
-  const T ptotstar = O::div(O::mad(rcl * rcr, ul - ur, rcr * ptotl + rcl * ptotr), rcr + rcl);
-
-  const bool left = ustar > T(0.0);
-  const T rk = left ? rl : rr;
-  const T uk = left ? ul : ur;
-  const T Sk = left ? SL : SR;
-  const T ek = left ? etotl : etotr;
-  const T pk = left ? ptotl : ptotr;
-  const T rstar = O::div(rk * (Sk - uk), Sk - ustar);
-  const T etotstar = O::div(O::mad(ptotstar, ustar, O::mad(-pk, uk, (Sk - uk) * ek)), Sk - ustar);
-
-  T ro, uo, ptoto, etoto;
-  if (SL > T(0.0)) {
-    ro = rl; uo = ul; ptoto = ptotl; etoto = etotl;
-  } else if (left || SR > T(0.0)) {
-    ro = rstar; uo = ustar; ptoto = ptotstar; etoto = etotstar;
+  const T pn = O::mad(rcl * rcr, ul - ur, rcr * pl + rcl * pr);
+  const T rc = rcr + rcl;
+  T ustar, ptotstar;
+  if constexpr (BND) {
+    const T r = recip_newton(rc);
+    ok = ok && rc >= T(0x1p-150);
+    ustar = quot_resid(un, rc, r, ok);
+    ptotstar = quot_plain(pn, rc, r);
   } else {
-    ro = rr; uo = ur; ptoto = ptotr; etoto = etotr;
+    ustar = O::div(un, rc);
+    ptotstar = O::div(pn, rc);
+  }
+
+  const bool upwind = SL > T(0.0);  // the whole fan moves right
+  const bool left = ustar > T(0.0);
+  const bool side = left || upwind;
+  const T rk = side ? rl : rr;
+  const T uk = side ? ul : ur;
+  const T pk = side ? pl : pr;
+  const T vk = side ? ql.v[tn] : qr.v[tn];
+  const T Sk = left ? SL : SR;
+  T ek = h * rk * uk * uk;
+  ek = O::mad(h * rk * vk, vk, ek);
+  ek = O::mad(pk, s.entho, ek);
+  T ro = rk, uo = uk, ptoto = pk, etoto = ek;
+  // FP32: a branch around the star state; its ends keep the compiler from
+  // interleaving the x and y fluxes of a row, which would cost the split step
+  // its third wavefront per SIMD (183 registers instead of 167)
+  if (sizeof(T) == sizeof(double) || !upwind) {
+    const T rn = rk * (Sk - uk);
+    const T en = O::mad(ptotstar, ustar, O::mad(-pk, uk, (Sk - uk) * ek));
+    const T sd = Sk - ustar;
+    T rstar, etotstar;
+    if constexpr (BND) {
+      const T r = recip_newton(sd);
+      ok = ok && O::ab(sd) >= T(0x1p-200);
+      rstar = quot_plain(rn, sd, r);
+      etotstar = quot_resid(en, sd, r, ok);
+    } else {
+      rstar = O::div(rn, sd);
+      etotstar = O::div(en, sd);
+    }
+    const bool star = !upwind && (left || SR > T(0.0));
+    ro = star ? rstar : rk;
+    uo = star ? ustar : uk;
+    ptoto = star ? ptotstar : pk;
+    etoto = star ? etotstar : ek;
   }
   const T fd = ro * uo;
   flux[ID] = fd;
@@ -482,24 +616,24 @@ __device__ __forceinline__ void hllc(const SchemeT<T> &s, const Q4T<T> &ql, cons
 
 // HLL (no reference counterpart; the reference declares the enum only,
 // HydroParams.h:49).  Toro 2009, section 10.3, eq. (10.21), with the floors and
-// wave speeds of riemann_hllc.  Same expressions as the CPU oracle.
-template <bool FS = false, class T>
+// wave speeds of riemann_hllc.  Same expressions as the CPU oracle.  BND: SR - SL
+// is at least 2^-113 wherever the middle state is taken, so its reciprocal needs
+// no test.
+template <bool FS = false, bool BND = false, class T>
 __device__ __forceinline__ void hll(const SchemeT<T> &s, const Q4T<T> &ql, const Q4T<T> &qr,
                                     int ln, int tn, T flux[4]) {
   using O = Ops<T>;
   const T h = T(0.5);
-  const T rl = O::mx(ql.v[ID], s.smallr);
+  const T rl = ql.v[ID], rr = qr.v[ID];  // floored by trace_face
   const T pl = O::mx(ql.v[IP], rl * s.smallp);
   const T ul = ql.v[ln], vl = ql.v[tn];
-  const T rr = O::mx(qr.v[ID], s.smallr);
   const T pr = O::mx(qr.v[IP], rr * s.smallp);
   const T ur = qr.v[ln], vr = qr.v[tn];
   const T el = O::mad(pl, s.entho, O::mad(h * rl * vl, vl, h * rl * ul * ul));
   const T er = O::mad(pr, s.entho, O::mad(h * rr * vr, vr, h * rr * ur * ur));
-  const T cfastl = floored_sqrt<FS>(O::mx(O::div(s.gamma0 * pl, rl), s.smallc2));
-  const T cfastr = floored_sqrt<FS>(O::mx(O::div(s.gamma0 * pr, rr), s.smallc2));
-  const T SL = O::mn(ul, ur) - O::mx(cfastl, cfastr);
-  const T SR = O::mx(ul, ur) + O::mx(cfastl, cfastr);
+  const T cmax = wave_speed<FS, BND>(s, pl, rl, pr, rr);
+  const T SL = O::mn(ul, ur) - cmax;
+  const T SR = O::mx(ul, ur) + cmax;
   // variable order of the conserved state: rho, E, normal momentum, transverse momentum
   const T UL[4] = {rl, el, rl * ul, rl * vl};
   const T UR[4] = {rr, er, rr * ur, rr * vr};
@@ -511,7 +645,11 @@ __device__ __forceinline__ void hll(const SchemeT<T> &s, const Q4T<T> &ql, const
   } else if (SR <= T(0.0)) {
     for (int k = 0; k < 4; k++) f[k] = FR[k];
   } else {
-    const T inv = O::div(T(1.0), SR - SL);
+    T inv;
+    if constexpr (BND)
+      inv = quot_plain(T(1.0), SR - SL, recip_newton(SR - SL));
+    else
+      inv = O::div(T(1.0), SR - SL);
     // SR*FL - SL*FR with separate products: exactly zero mass flux for
     // mirrored states at a reflecting wall
     for (int k = 0; k < 4; k++)
@@ -613,17 +751,26 @@ constexpr int kMinmodPow2 = 16;
 // batch kernels, whose instances' cell sizes may be anything)
 constexpr int kSlopeMinmod = 32;
 
-template <int RS, class T>
+// BND: the states are in the bounded ranges; ok is cleared in a lane whose flux
+// may not have the IEEE bits
+template <int RS, bool BND, class T>
 __device__ __forceinline__ void riemann(const SchemeT<T> &s, const Q4T<T> &ql, const Q4T<T> &qr,
-                                        int ln, int tn, T flux[4]) {
+                                        int ln, int tn, T flux[4], bool &ok) {
   constexpr int kind = RS & 7;
   constexpr bool fs = (RS & kRiemannFloorSqrt) != 0;
   if constexpr (kind == 2)
-    hllc<fs>(s, ql, qr, ln, tn, flux);
+    hllc<fs, BND>(s, ql, qr, ln, tn, flux, ok);
   else if constexpr (kind == 1)
-    hll<fs>(s, ql, qr, ln, tn, flux);
+    hll<fs, BND>(s, ql, qr, ln, tn, flux);
   else
     approx(s, ql, qr, ln, tn, flux);
+}
+
+template <int RS, class T>
+__device__ __forceinline__ void riemann(const SchemeT<T> &s, const Q4T<T> &ql, const Q4T<T> &qr,
+                                        int ln, int tn, T flux[4]) {
+  bool ok = true;
+  riemann<RS, false>(s, ql, qr, ln, tn, flux, ok);
 }
 
 }  // namespace e2d
