@@ -13,6 +13,9 @@
 #include <cstring>
 #include <new>
 #include <string>
+#include <system_error>
+#include <thread>
+#include <utility>
 #include <vector>
 
 #include <cmath>
@@ -73,6 +76,15 @@ struct e2d_config {
   e2d::ConfigMap map;
 };
 
+// Pinned buffers of host copies (`nbuf` of `bytes` each) and an event per buffer,
+// made by the first copy that needs them.
+struct Staging {
+  char *host = nullptr;
+  size_t bytes = 0;
+  int nbuf = 0;
+  hipEvent_t ev[8] = {};
+};
+
 struct e2d_run {
   e2d_params p{};
   e2d::KParams kp{};
@@ -95,6 +107,7 @@ struct e2d_run {
   double *sums4 = nullptr;
   double timers[5] = {0, 0, 0, 0, 0};
   std::vector<void *> allocs;
+  Staging staging;  // host copies
 };
 
 namespace {
@@ -132,6 +145,15 @@ int check_run(e2d_run *r) {
   if (!r) return fail(E2D_ERR_ARG, "null e2d_run handle");
   hipError_t e = hipSetDevice(r->device);
   if (e != hipSuccess) return hip_fail(e, "hipSetDevice");
+  return E2D_OK;
+}
+
+int check_copy(e2d_run *r, int which, const double *host, int layout) {
+  const int rc = check_run(r);
+  if (rc) return rc;
+  if (!host || (which != E2D_U && which != E2D_U2)) return fail(E2D_ERR_ARG, "bad argument");
+  if (layout != E2D_LAYOUT_INTERIOR && layout != E2D_LAYOUT_LEFT && layout != E2D_LAYOUT_RIGHT)
+    return fail(E2D_ERR_ARG, "unknown layout");
   return E2D_OK;
 }
 
@@ -435,103 +457,117 @@ int run_loop_impl(e2d_run *r, int max_steps, double *t, int *nStep, double *elap
   return E2D_OK;
 }
 
-// Device state -> host FP64 planes [v][j][i] (isize x jsize, ghosts included);
-// the split representation is combined as (double)hi + (double)lo.
-int download_planes(e2d_run *r, const Grid &g, std::vector<double> &out) {
-  const int isz = r->p.isize, jsz = r->p.jsize;
-  const size_t cells = (size_t)isz * jsz;
-  out.assign(4 * cells, 0.0);
-  if (r->precision == E2D_PRECISION_FP64) {
-    const double *src = static_cast<const double *>(g.p);
-    for (int v = 0; v < 4; v++)
-      HIP_TRY(hipMemcpy2DAsync(out.data() + v * cells, (size_t)isz * sizeof(double),
-                               src + v * g.plane, (size_t)g.pitch * sizeof(double),
-                               (size_t)isz * sizeof(double), (size_t)jsz, hipMemcpyDeviceToHost,
-                               r->stream));
-    HIP_TRY(hipStreamSynchronize(r->stream));
-    return E2D_OK;
-  }
-  // split: (hi, lo) float pairs; FP32: floats
-  const int per = r->precision == E2D_PRECISION_FP32_SPLIT ? 2 : 1;
-  const size_t eb = per * sizeof(float);
-  std::vector<float> tmp((size_t)per * 4 * cells);
-  const char *src = static_cast<const char *>(g.p);
-  for (int v = 0; v < 4; v++)
-    HIP_TRY(hipMemcpy2DAsync(tmp.data() + (size_t)per * v * cells, (size_t)isz * eb,
-                             src + (size_t)v * g.plane * eb, (size_t)g.pitch * eb, (size_t)isz * eb,
-                             (size_t)jsz, hipMemcpyDeviceToHost, r->stream));
-  HIP_TRY(hipStreamSynchronize(r->stream));
-  for (size_t k = 0; k < 4 * cells; k++)
-    out[k] = per == 2 ? (double)tmp[2 * k] + (double)tmp[2 * k + 1] : (double)tmp[k];
-  return E2D_OK;
-}
+// Bytes of one staging chunk.  A copy goes chunk by chunk through pinned
+// buffers, two per host thread: while a thread copies one to (from) the caller's
+// array, the GPU fills (empties) the other.  Smaller chunks pay a launch and a
+// wait (about 10 us) too often, larger ones leave more of the first and last
+// chunk unoverlapped.
+constexpr size_t kStageChunk = 2u << 20;
+// From 16 MiB on, four threads copy: one alone moves 13 GB/s into memory that the
+// caller has just allocated (page faults), PCIe about 50 GB/s.  A 1024x1536 state
+// (50 MB) takes 3.8 ms with one thread and 2.0 ms with four (57 ms as plane copies
+// followed by a host loop over the layout); below the line, where one chunk or a
+// few make up the copy, threads bring nothing (8.5 MB: 0.38 ms either way).
+constexpr int kStageThreads = 4;
+constexpr size_t kStageThreadsFrom = 16u << 20;
 
-// Host FP64 planes -> device state (split: hi = (float)x, lo = (float)(x - hi)).
-int upload_planes(e2d_run *r, const Grid &g, const std::vector<double> &in) {
-  const int isz = r->p.isize, jsz = r->p.jsize;
-  const size_t cells = (size_t)isz * jsz;
-  if (r->precision == E2D_PRECISION_FP64) {
-    double *dst = static_cast<double *>(g.p);
-    for (int v = 0; v < 4; v++)
-      HIP_TRY(hipMemcpy2DAsync(dst + v * g.plane, (size_t)g.pitch * sizeof(double),
-                               in.data() + v * cells, (size_t)isz * sizeof(double),
-                               (size_t)isz * sizeof(double), (size_t)jsz, hipMemcpyHostToDevice,
-                               r->stream));
-    HIP_TRY(hipStreamSynchronize(r->stream));
-    return E2D_OK;
-  }
-  const int per = r->precision == E2D_PRECISION_FP32_SPLIT ? 2 : 1;
-  const size_t eb = per * sizeof(float);
-  std::vector<float> tmp((size_t)per * 4 * cells);
-  for (size_t k = 0; k < 4 * cells; k++) {
-    const double x = in[k];
-    const float hi = (float)x;
-    if (per == 2) {
-      tmp[2 * k] = hi;
-      tmp[2 * k + 1] = (float)(x - (double)hi);
-    } else {
-      tmp[k] = hi;
+// `nbuf` pinned buffers of at least `bytes` bytes, with an event each
+hipError_t stage_reserve(Staging &s, size_t bytes, int nbuf) {
+  for (int k = 0; k < nbuf; ++k)
+    if (!s.ev[k]) {
+      const hipError_t e = hipEventCreateWithFlags(&s.ev[k], hipEventDisableTiming);
+      if (e != hipSuccess) return e;
     }
+  if (s.bytes >= bytes && s.nbuf >= nbuf) return hipSuccess;
+  if (s.host) (void)hipHostFree(s.host);
+  s.host = nullptr;
+  s.bytes = 0;
+  s.nbuf = 0;
+  void *p = nullptr;
+  const hipError_t e = hipHostMalloc(&p, bytes * nbuf, hipHostMallocDefault);
+  if (e != hipSuccess) return e;
+  s.host = static_cast<char *>(p);
+  s.bytes = bytes;
+  s.nbuf = nbuf;
+  return hipSuccess;
+}
+
+void stage_release(Staging &s) {
+  for (hipEvent_t e : s.ev)
+    if (e) (void)hipEventDestroy(e);
+  if (s.host) (void)hipHostFree(s.host);
+  s = Staging{};
+}
+
+// State array <-> host array in one of the E2D_LAYOUT_* layouts.  The whole
+// copy is done when this returns.
+int stage_copy(const e2d_run *r, Staging &s, const Grid &g, double *host, int layout,
+               bool to_host) {
+  const e2d_params &p = r->p;
+  const e2d::HostBox box = layout == E2D_LAYOUT_INTERIOR ? e2d::HostBox{2, 2, p.nx, p.ny}
+                                                         : e2d::HostBox{0, 0, p.isize, p.jsize};
+  const bool columns = layout == E2D_LAYOUT_RIGHT;
+  const int units = columns ? box.ni : 4 * box.nj;
+  const size_t unit = columns ? (size_t)box.nj * 32 : (size_t)box.ni * 8;
+  int per = (int)std::min<size_t>((size_t)units, std::max<size_t>(1, kStageChunk / unit));
+  if (columns && per < units && per > 16) per -= per % 16;  // whole tiles
+  const int nchunks = (units + per - 1) / per;
+  const int nthreads = unit * units >= kStageThreadsFrom ? std::min(kStageThreads, nchunks) : 1;
+  const hipError_t re = stage_reserve(s, unit * per, nchunks > 1 ? 2 * nthreads : 1);
+  if (re != hipSuccess)
+    return fail(E2D_ERR_ALLOC, std::string("staging buffers: ") + hipGetErrorString(re));
+
+  // thread t moves chunks t, t + nthreads, ... through its two buffers
+  auto worker = [&](int t) -> hipError_t {
+    hipError_t e = hipSetDevice(r->device);
+    auto count = [&](int k) { return std::min(per, units - k * per); };
+    auto user = [&](int k) { return reinterpret_cast<char *>(host) + (size_t)k * per * unit; };
+    int before = -1;  // the chunk in the other buffer
+    for (int k = t, n = 0; e == hipSuccess && k < nchunks; k += nthreads, ++n) {
+      const int slot = 2 * t + (n & 1);
+      char *buf = s.host + (size_t)slot * s.bytes;
+      if (!to_host) {
+        if (n > 1) e = hipEventSynchronize(s.ev[slot]);  // its last chunk has left the buffer
+        if (e != hipSuccess) break;
+        std::memcpy(buf, user(k), count(k) * unit);
+      }
+      e = e2d::launch_staging(r->precision, g, box, columns, k * per, count(k),
+                              reinterpret_cast<double *>(buf), to_host, r->stream);
+      if (e == hipSuccess) e = hipEventRecord(s.ev[slot], r->stream);
+      if (to_host && before >= 0 && e == hipSuccess) {
+        e = hipEventSynchronize(s.ev[slot ^ 1]);
+        if (e == hipSuccess)
+          std::memcpy(user(before), s.host + (size_t)(slot ^ 1) * s.bytes, count(before) * unit);
+      }
+      before = k;
+      if (to_host && k + nthreads >= nchunks && e == hipSuccess) {  // this thread's last chunk
+        e = hipEventSynchronize(s.ev[slot]);
+        if (e == hipSuccess) std::memcpy(user(k), buf, count(k) * unit);
+      }
+    }
+    return e;
+  };
+
+  hipError_t err[kStageThreads] = {};
+  std::thread helpers[kStageThreads];
+  int mine = 1;  // chunk sequences 0 .. mine - 1 and those no thread could be started for
+  for (int t = 1; t < nthreads; ++t) {
+    try {
+      helpers[t] = std::thread([&, t] { err[t] = worker(t); });
+    } catch (const std::system_error &) {
+      break;
+    }
+    mine = t + 1;
   }
-  char *dst = static_cast<char *>(g.p);
-  for (int v = 0; v < 4; v++)
-    HIP_TRY(hipMemcpy2DAsync(dst + (size_t)v * g.plane * eb, (size_t)g.pitch * eb,
-                             tmp.data() + (size_t)per * v * cells, (size_t)isz * eb,
-                             (size_t)isz * eb, (size_t)jsz, hipMemcpyHostToDevice, r->stream));
-  HIP_TRY(hipStreamSynchronize(r->stream));
+  err[0] = worker(0);
+  for (int t = mine; t < nthreads; ++t) err[t] = worker(t);
+  for (std::thread &h : helpers)
+    if (h.joinable()) h.join();
+  const hipError_t se = hipStreamSynchronize(r->stream);
+  for (hipError_t e : err)
+    if (e != hipSuccess) return hip_fail(e, "host copy");
+  if (se != hipSuccess) return hip_fail(se, "host copy");
   return E2D_OK;
-}
-
-void planes_to_layout(const e2d_run *r, const std::vector<double> &pl, double *host, int layout) {
-  const int isz = r->p.isize, jsz = r->p.jsize, nx = r->p.nx, ny = r->p.ny;
-  const size_t cells = (size_t)isz * jsz;
-  for (int v = 0; v < 4; v++)
-    for (int j = 0; j < jsz; j++)
-      for (int i = 0; i < isz; i++) {
-        const double x = pl[v * cells + (size_t)j * isz + i];
-        if (layout == E2D_LAYOUT_RIGHT)
-          host[((size_t)i * jsz + j) * 4 + v] = x;
-        else if (layout == E2D_LAYOUT_LEFT)
-          host[v * cells + (size_t)j * isz + i] = x;
-        else if (i >= 2 && i < nx + 2 && j >= 2 && j < ny + 2)
-          host[(size_t)v * nx * ny + (size_t)(j - 2) * nx + (i - 2)] = x;
-      }
-}
-
-void layout_to_planes(const e2d_run *r, const double *host, int layout, std::vector<double> &pl) {
-  const int isz = r->p.isize, jsz = r->p.jsize, nx = r->p.nx, ny = r->p.ny;
-  const size_t cells = (size_t)isz * jsz;
-  for (int v = 0; v < 4; v++)
-    for (int j = 0; j < jsz; j++)
-      for (int i = 0; i < isz; i++) {
-        double &x = pl[v * cells + (size_t)j * isz + i];
-        if (layout == E2D_LAYOUT_RIGHT)
-          x = host[((size_t)i * jsz + j) * 4 + v];
-        else if (layout == E2D_LAYOUT_LEFT)
-          x = host[v * cells + (size_t)j * isz + i];
-        else if (i >= 2 && i < nx + 2 && j >= 2 && j < ny + 2)
-          x = host[(size_t)v * nx * ny + (size_t)(j - 2) * nx + (i - 2)];
-      }
 }
 
 template <class F>
@@ -755,6 +791,7 @@ int e2d_destroy(e2d_run *run) {
   if (run->ev0) (void)hipEventDestroy(run->ev0);
   if (run->ev1) (void)hipEventDestroy(run->ev1);
   if (run->host_s) (void)hipHostFree(run->host_s);
+  stage_release(run->staging);
   for (void *ptr : run->allocs) (void)hipFree(ptr);
   if (run->stream) (void)hipStreamDestroy(run->stream);
   delete run;
@@ -839,39 +876,19 @@ int e2d_time_loop(e2d_run *r, int nsteps, double *elapsed_ms, int *executed, dou
 }
 
 int e2d_copy_state(e2d_run *r, int which, double *host, int layout) {
-  int rc = check_run(r);
+  const int rc = check_copy(r, which, host, layout);
   if (rc) return rc;
-  if (!host || (which != E2D_U && which != E2D_U2)) return fail(E2D_ERR_ARG, "bad argument");
-  if (layout != E2D_LAYOUT_INTERIOR && layout != E2D_LAYOUT_LEFT && layout != E2D_LAYOUT_RIGHT)
-    return fail(E2D_ERR_ARG, "unknown layout");
-  const Grid &g = state(r, which);
   return guarded([&]() -> int {
-    std::vector<double> planes;
-    rc = download_planes(r, g, planes);
-    if (rc) return rc;
-    planes_to_layout(r, planes, host, layout);
-    return E2D_OK;
+    return stage_copy(r, r->staging, state(r, which), host, layout, true);
   });
 }
 
 int e2d_upload_state(e2d_run *r, int which, const double *host, int layout) {
-  int rc = check_run(r);
+  const int rc = check_copy(r, which, host, layout);
   if (rc) return rc;
-  if (!host || (which != E2D_U && which != E2D_U2)) return fail(E2D_ERR_ARG, "bad argument");
-  if (layout != E2D_LAYOUT_INTERIOR && layout != E2D_LAYOUT_LEFT && layout != E2D_LAYOUT_RIGHT)
-    return fail(E2D_ERR_ARG, "unknown layout");
-  const Grid &g = state(r, which);
+  // an interior copy leaves the ghost cells that the device holds
   return guarded([&]() -> int {
-    std::vector<double> planes;
-    if (layout == E2D_LAYOUT_INTERIOR) {
-      // keep the ghost cells the device already holds
-      rc = download_planes(r, g, planes);
-      if (rc) return rc;
-    } else {
-      planes.assign((size_t)4 * r->p.isize * r->p.jsize, 0.0);
-    }
-    layout_to_planes(r, host, layout, planes);
-    return upload_planes(r, g, planes);
+    return stage_copy(r, r->staging, state(r, which), const_cast<double *>(host), layout, false);
   });
 }
 
@@ -1125,6 +1142,9 @@ struct e2d_batch {
   e2d::BatchQueue queue{};
   std::vector<int> queue_per_step;       // host copy of queue.per_step
   e2d::BatchCounters *counters = nullptr;  // device, followed by done[count * kCounterStride]
+  Staging staging;  // host copies of every instance's state
+  // the instances' loop states as e2d_batch_run read them at its end (empty: not read)
+  std::vector<e2d::StepState> states;
 };
 
 namespace {
@@ -1276,8 +1296,13 @@ int batch_graph(e2d_batch *b) {
 
 // state of instance i after the launched steps
 int batch_state(e2d_batch *b, int i, e2d::StepState &s) {
+  if (!b->states.empty()) {
+    s = b->states[(size_t)i];
+    return E2D_OK;
+  }
   HIP_TRY(hipMemcpyAsync(&s, &b->ctls[i].s[b->phase], sizeof(s), hipMemcpyDeviceToHost,
                          b->stream));
+  HIP_TRY(hipStreamSynchronize(b->stream));
   return E2D_OK;
 }
 
@@ -1291,6 +1316,7 @@ int batch_active(e2d_batch *b, int *active) {
   int n = 0;
   for (size_t i = 0; i < s.size(); ++i) n += loop_view(b->runs[i]->p, s[i]).active ? 1 : 0;
   *active = n;
+  b->states = std::move(s);
   return E2D_OK;
 }
 
@@ -1488,6 +1514,7 @@ int e2d_batch_destroy(e2d_batch *b) {
   if (b->stream) (void)hipStreamSynchronize(b->stream);
   batch_drop_graph(b);
   for (e2d_run *r : b->runs) e2d_destroy(r);
+  stage_release(b->staging);
   if (b->insts) (void)hipFree(b->insts);
   if (b->ctls) (void)hipFree(b->ctls);
   if (b->queue_ints) (void)hipFree(b->queue_ints);
@@ -1502,6 +1529,7 @@ int e2d_batch_init(e2d_batch *b) {
   if (rc) return rc;
   // phase 0 of every instance's rings: t = 0, nStep = 0, the rest cleared
   b->ready = false;
+  b->states.clear();
   b->phase = 0;
   HIP_TRY(hipMemsetAsync(b->ctls, 0, sizeof(e2d::StepCtl) * b->runs.size(), b->stream));
   HIP_TRY(hipStreamSynchronize(b->stream));
@@ -1532,6 +1560,7 @@ int e2d_batch_run(e2d_batch *b, int max_steps, int use_graph, double *elapsed_ms
   if (rc) return rc;
   if (max_steps <= 0) return fail(E2D_ERR_ARG, "max_steps must be > 0");
   if (!b->ready) return fail(E2D_ERR_ARG, "e2d_batch_init has not run on this batch");
+  b->states.clear();
   if (b->launch == E2D_BATCH_LAUNCH_PERSISTENT) return batch_run_persistent(b, max_steps,
                                                                             elapsed_ms, active_left);
   if (use_graph) {
@@ -1571,7 +1600,6 @@ int e2d_batch_status(e2d_batch *b, int instance, double *t, int *nStep) {
   e2d::StepState s{};
   rc = batch_state(b, instance, s);
   if (rc) return rc;
-  HIP_TRY(hipStreamSynchronize(b->stream));
   if (t) *t = s.t;
   if (nStep) *nStep = s.nstep;
   return E2D_OK;
@@ -1582,7 +1610,12 @@ int e2d_batch_copy_state(e2d_batch *b, int instance, double *host, int layout) {
   int n = 0;
   int rc = e2d_batch_status(b, instance, &t, &n);
   if (rc) return rc;
-  return e2d_copy_state(b->runs[instance], n % 2 == 0 ? E2D_U : E2D_U2, host, layout);
+  e2d_run *r = b->runs[instance];
+  const int which = n % 2 == 0 ? E2D_U : E2D_U2;
+  if ((rc = check_copy(r, which, host, layout))) return rc;
+  return guarded([&]() -> int {
+    return stage_copy(r, b->staging, state(r, which), host, layout, true);
+  });
 }
 
 int e2d_batch_info(e2d_batch *b, long long *cells, int *waves, int *count) {

@@ -117,6 +117,12 @@ struct RadialGeom {
   int nbins;
 };
 
+// Cells of a state array that a host copy holds: columns i0 .. i0 + ni - 1 of
+// rows j0 .. j0 + nj - 1, every variable.
+struct HostBox {
+  int i0, j0, ni, nj;
+};
+
 // fused step geometry: one wave of 64 lanes covers 60 output columns (plus a
 // 2-column halo on each side) and marches over `seg_rows` output rows
 constexpr int kLanes = 64;
@@ -207,6 +213,11 @@ hipError_t launch_xcc_probe(unsigned *out, int blocks, hipStream_t st);
 // per-bin cell counts and density sums of the radial profile (nbins entries each)
 hipError_t launch_radial_profile(const KParams &kp, Grid U, const RadialGeom &geo,
                                  unsigned long long *counts, double *sums, hipStream_t st);
+// Part of a state array to (to_host) or from pinned host memory as FP64 values:
+// `units` units from `first` on, the first at host[0].  Units are the box's
+// rows in [var][j][i] order or, with `columns`, its columns in [i][j][var] order.
+hipError_t launch_staging(int precision, Grid g, const HostBox &b, bool columns, int first,
+                          int units, double *host, bool to_host, hipStream_t st);
 // *p = v, one thread (a kernel, so that it may be captured in a graph)
 hipError_t launch_fill_u32(unsigned *p, unsigned v, hipStream_t st);
 // whole-array copy (all planes, ghosts and padding included)

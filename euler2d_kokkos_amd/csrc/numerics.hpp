@@ -741,7 +741,8 @@ __device__ __forceinline__ void approx(const SchemeT<T> &s, const Q4T<T> &qlf, c
 
 // solver chosen at compile time: RS = 0 approx, 1 hll, 2 hllc
 // RS: 0 approx, 1 HLL, 2 HLLC; + kRiemannFloorSqrt: the HLL/HLLC wave speeds
-// use the short square root (FP64, arguments floored at smallc^2 >= 2^-759)
+// use the short square root and, in the march, the bounded quotients (FP64,
+// where SchemeT::floor_sqrt holds)
 constexpr int kRiemannFloorSqrt = 8;
 // + kMinmodPow2: the march is built for slope_type == 1 (its slopes) and for
 // cell sizes that are powers of two (its CFL rate); the host selects such a
