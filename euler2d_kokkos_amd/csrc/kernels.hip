@@ -400,14 +400,49 @@ __device__ __forceinline__ unsigned long long dbits(double x) {
   return (unsigned long long)__double_as_longlong(x);
 }
 
-__device__ __forceinline__ double wave_max(double x) {
-  for (int off = 32; off > 0; off >>= 1) x = fmax(x, __shfl_xor(x, off));
-  return x;
+// DPP controls: row_ror:n rotates within each row of 16 lanes
+constexpr int kDppRowRor1 = 0x121, kDppRowRor2 = 0x122, kDppRowRor4 = 0x124, kDppRowRor8 = 0x128;
+
+template <int CTRL>
+__device__ __forceinline__ float dpp_shift(float x) {
+  const int v = __float_as_int(x);
+  return __int_as_float(__builtin_amdgcn_mov_dpp(v, CTRL, 0xf, 0xf, true));
 }
 
-__device__ __forceinline__ float wave_max(float x) {
-  for (int off = 32; off > 0; off >>= 1) x = fmaxf(x, __shfl_xor(x, off));
-  return x;
+template <int CTRL>
+__device__ __forceinline__ double dpp_shift(double x) {
+  const long long b = __double_as_longlong(x);
+  const int lo = (int)(b & 0xffffffffll), hi = (int)(b >> 32);
+  const int rlo = __builtin_amdgcn_mov_dpp(lo, CTRL, 0xf, 0xf, true);
+  const int rhi = __builtin_amdgcn_mov_dpp(hi, CTRL, 0xf, 0xf, true);
+  return __longlong_as_double(((long long)rhi << 32) | (unsigned int)rlo);
+}
+
+__device__ __forceinline__ double lane_value(double x, int lane) {
+  const long long b = __double_as_longlong(x);
+  const unsigned lo = (unsigned)__builtin_amdgcn_readlane((int)b, lane);
+  const unsigned hi = (unsigned)__builtin_amdgcn_readlane((int)(b >> 32), lane);
+  return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
+}
+
+// Max over each row of 16 lanes, in every lane of the row: four lane rotations
+// (full-rate moves).  All lanes must be active.  The reduction sits on the
+// serial head and tail of every step, where the LDS-routed shuffles it replaced
+// took about 0.3 us each.
+template <class T>
+__device__ __forceinline__ T row_max(T x) {
+  x = Ops<T>::mx(x, dpp_shift<kDppRowRor8>(x));
+  x = Ops<T>::mx(x, dpp_shift<kDppRowRor4>(x));
+  x = Ops<T>::mx(x, dpp_shift<kDppRowRor2>(x));
+  return Ops<T>::mx(x, dpp_shift<kDppRowRor1>(x));
+}
+
+// max over the wavefront, the same value in every lane
+template <class T>
+__device__ __forceinline__ double wave_max(T x) {
+  const double r = (double)row_max(x);
+  return fmax(fmax(lane_value(r, 0), lane_value(r, 16)),
+              fmax(lane_value(r, 32), lane_value(r, 48)));
 }
 
 // ------------------------------------------------------------------ init
@@ -550,7 +585,7 @@ __global__ __launch_bounds__(256) void dt_reduce_kernel(KParams kp, Grid U,
   // block max, then one device-scope atomic per block (the max is exact and
   // order independent)
   __shared__ double wm[256 / kLanes];
-  const double md = (double)wave_max(m);
+  const double md = wave_max(m);
   if ((threadIdx.x & (kLanes - 1)) == 0) wm[threadIdx.x / kLanes] = md;
   __syncthreads();
   if (threadIdx.x == 0) {
@@ -636,7 +671,7 @@ __global__ __launch_bounds__(kBeginThreads) void loop_begin_kernel(KParams kp, G
     }
   __shared__ double wm[kBeginThreads / kLanes];
   __shared__ bool last;
-  const double md = (double)wave_max(m);
+  const double md = wave_max(m);
   if ((threadIdx.x & (kLanes - 1)) == 0) wm[threadIdx.x / kLanes] = md;
   __syncthreads();
   if (threadIdx.x == 0) {
@@ -892,21 +927,6 @@ __global__ void fluxes_atomic_kernel(KParams kp, Grid Q, Grid U, double dtdx, do
 constexpr int kDppWaveRor1 = 0x13c;  // lane i reads lane i-1, lane 0 lane 63
 constexpr int kDppWaveRol1 = 0x134;  // lane i reads lane i+1, lane 63 lane 0
 
-template <int CTRL>
-__device__ __forceinline__ float dpp_shift(float x) {
-  const int v = __float_as_int(x);
-  return __int_as_float(__builtin_amdgcn_mov_dpp(v, CTRL, 0xf, 0xf, true));
-}
-
-template <int CTRL>
-__device__ __forceinline__ double dpp_shift(double x) {
-  const long long b = __double_as_longlong(x);
-  const int lo = (int)(b & 0xffffffffll), hi = (int)(b >> 32);
-  const int rlo = __builtin_amdgcn_mov_dpp(lo, CTRL, 0xf, 0xf, true);
-  const int rhi = __builtin_amdgcn_mov_dpp(hi, CTRL, 0xf, 0xf, true);
-  return __longlong_as_double(((long long)rhi << 32) | (unsigned int)rlo);
-}
-
 template <class T>
 __device__ __forceinline__ Q4T<T> shfl_up1(const Q4T<T> &a) {
   Q4T<T> r;
@@ -1154,10 +1174,12 @@ __device__ __forceinline__ void set_prio_level(int lvl) {
     __builtin_amdgcn_s_setprio(0);
 }
 
-template <int RS, class P, bool RATE, bool O32, bool COLS, int PD>
+// `start` gives dt and whether the step runs at all.  It is asked after the first
+// rows' loads are issued, so that their latency overlaps its own.
+template <int RS, class P, bool RATE, bool O32, bool COLS, int PD, class Start>
 __device__ __forceinline__ typename P::T march(const KParams &kp, const Grid &in, const Grid &out,
-                                               double dt, int seg_rows, int nstrips, int strip,
-                                               int seg, bool prio, bool go = true) {
+                                               Start &&start, int seg_rows, int nstrips,
+                                               int strip, int seg, bool prio) {
   using T = typename P::T;
   const int lane = threadIdx.x & (kLanes - 1);
 
@@ -1201,9 +1223,8 @@ __device__ __forceinline__ typename P::T march(const KParams &kp, const Grid &in
     }
     if (flipy) P::negate(dst, IV);
   }
-  // go = false (run loop ended): nothing is stored.  The check comes after the
-  // first row's load is issued, so that its latency overlaps the loop-state read.
-  if (!go) return T(0.0);
+  double dt;
+  if (!start(dt)) return T(0.0);  // run loop ended: nothing is stored
   const T dtdx = (T)(dt / kp.dx);
   const T dtdy = (T)(dt / kp.dy);
   m.ua = m.un;
@@ -1281,25 +1302,42 @@ struct LoopPos {
   bool active;
 };
 
-__device__ __forceinline__ LoopPos loop_pos(const KParams &kp, const StepCtl *ctl, int ph) {
-  LoopPos L;
-  L.t = ctl->s[ph].t;
-  L.nstep = ctl->s[ph].nstep;
-  L.active = L.t < kp.tEnd && L.nstep < kp.nStepmax;
-  // one vector load reads the 16 slots (16 lines) at once: lane k reads slot k.
-  // The slots hold +0 or positive rates, so the max of the doubles is the max
-  // of their bits.
+// The words of launch phase ph: one vector load reads the 16 slots (16 lines) at
+// once, lane k slot k.  The caller issues its first row loads between the two
+// halves, so that one memory round trip covers both.
+struct LoopWords {
+  double t, slot;
+  int nstep;
+};
+
+__device__ __forceinline__ LoopWords loop_words(const StepCtl *ctl, int ph) {
   const int lane = threadIdx.x & (kLanes - 1);
-  const double b =
-      lane < kRateSlots ? __longlong_as_double((long long)ctl->rate[ph][lane * kSlotStride]) : 0.0;
-  const long long mb = __double_as_longlong(wave_max(b));
-  const unsigned mlo = __builtin_amdgcn_readfirstlane((unsigned)mb);
-  const unsigned mhi = __builtin_amdgcn_readfirstlane((unsigned)(mb >> 32));
-  const double invdt = __longlong_as_double((long long)(((unsigned long long)mhi << 32) | mlo));
+  return LoopWords{ctl->s[ph].t,
+                   lane < kRateSlots
+                       ? __longlong_as_double((long long)ctl->rate[ph][lane * kSlotStride])
+                       : 0.0,
+                   ctl->s[ph].nstep};
+}
+
+// dt from the time before the step and the slots' values in lanes 0 .. 15 (+0
+// or positive rates)
+__device__ __forceinline__ LoopPos loop_resolve(const KParams &kp, double t, int nstep,
+                                                double slot) {
+  static_assert(kRateSlots == 16, "the slots fill one row of lanes");
+  LoopPos L;
+  L.t = t;
+  L.nstep = nstep;
+  L.active = L.t < kp.tEnd && L.nstep < kp.nStepmax;
+  const double invdt = lane_value(row_max(slot), 0);
   double dt = kp.cfl / invdt;
   if (L.t + dt > kp.tEnd) dt = kp.tEnd - L.t;
   L.dt = dt;
   return L;
+}
+
+__device__ __forceinline__ LoopPos loop_pos(const KParams &kp, const StepCtl *ctl, int ph) {
+  const LoopWords w = loop_words(ctl, ph);
+  return loop_resolve(kp, w.t, w.nstep, w.slot);
 }
 
 // The step's one writer, the lanes of one wavefront: the state after the step
@@ -1334,7 +1372,7 @@ __device__ __forceinline__ unsigned long long *rate_slot(StepCtl *ctl, int ph) {
 // A NaN rate never reaches a slot (m > 0 is false for it).
 template <class T>
 __device__ __forceinline__ void reduce_rate_wave(T wmax, unsigned long long *target) {
-  const double m = (double)wave_max(wmax);
+  const double m = wave_max(wmax);
   if ((threadIdx.x & (kLanes - 1)) == 0 && target && m > 0.0) atomicMax(target, dbits(m));
 }
 
@@ -1373,37 +1411,245 @@ void step_fused_kernel(KParams kp, Grid in, Grid out,
                                                             double dt_arg, StepCtl *ctl, int ph,
                                                             FusedMap fm) {
   using T = typename P::T;
-  double dt = dt_arg;
-  bool go = true;
-  if constexpr (LOOP) {
-    const LoopPos L = loop_pos(kp, ctl, ph);
-    if (blockIdx.x == 0 && threadIdx.x < kLanes) loop_publish(ctl, ph, L, threadIdx.x);
-    go = L.active;  // false once the loop has finished (uniform over the grid)
-    dt = L.dt;
-  }
   // the wave index is uniform: every row index and the row ghost map derived
   // from it are then scalar values and scalar control flow
   const int wave =
       __builtin_amdgcn_readfirstlane(blockIdx.x * (kBlock / kLanes) + (threadIdx.x >> 6));
-  T wmax = T(0.0);
-  if (wave < fm.nwaves) {
-    int strip, seg, tile;
-    fused_wave(fm, wave, strip, seg, tile);
-    // in and out share their geometry (checked at launch): one pitch and one
-    // plane stride let a row's offset serve both arrays
-    Grid o = in;
-    o.p = out.p;
-    if (interior_cols(kp, strip))  // uniform
-      wmax = march<RS, P, LOOP, O32, false, PD>(kp, in, o, dt, tile, fm.nstrips, strip, seg,
-                                            fm.prio != 0, go);
-    else
-      wmax = march<RS, P, LOOP, O32, true, PD>(kp, in, o, dt, tile, fm.nstrips, strip, seg,
-                                           fm.prio != 0, go);
-  }
+  if (wave >= fm.nwaves) return;  // (wavefront 0, which publishes, always marches)
+  LoopWords words;
+  if constexpr (LOOP) words = loop_words(ctl, ph);
+  bool go = true;
+  auto start = [&](double &dt) -> bool {
+    if constexpr (LOOP) {
+      const LoopPos L = loop_resolve(kp, words.t, words.nstep, words.slot);
+      if (wave == 0) loop_publish(ctl, ph, L, threadIdx.x & (kLanes - 1));
+      go = L.active;  // false once the loop has finished (uniform over the grid)
+      dt = L.dt;
+    } else {
+      dt = dt_arg;
+    }
+    return go;
+  };
+  int strip, seg, tile;
+  fused_wave(fm, wave, strip, seg, tile);
+  // in and out share their geometry (checked at launch): one pitch and one
+  // plane stride let a row's offset serve both arrays
+  Grid o = in;
+  o.p = out.p;
+  T wmax;
+  if (interior_cols(kp, strip))  // uniform
+    wmax = march<RS, P, LOOP, O32, false, PD>(kp, in, o, start, tile, fm.nstrips, strip, seg,
+                                              fm.prio != 0);
+  else
+    wmax = march<RS, P, LOOP, O32, true, PD>(kp, in, o, start, tile, fm.nstrips, strip, seg,
+                                             fm.prio != 0);
   // run loop: the CFL rate of the step's output, for the next launch's dt
   if constexpr (LOOP) {
-    if (!go) return;
-    reduce_rate_wave(wmax, rate_slot(ctl, ph));
+    if (go) reduce_rate_wave(wmax, rate_slot(ctl, ph));
+  }
+}
+
+// ------------------------------------------------------- block step kernel
+//
+// The step for small grids.  There the march is a serial chain: a wavefront
+// converts, slopes and traces row after row, four of them warm-up rows, at the
+// issue rate of one wavefront, while most of the chip is idle.  Here a block of
+// W wavefronts owns R = K W - 4 output rows of a strip and each wavefront K of
+// its K W loaded rows (one or two): it converts them, exchanges primitives, upper
+// face states and y fluxes with the wavefronts above and below through LDS,
+// forms the x fluxes with lane shifts and updates its rows.  The chain is K
+// rows', and all of a block's loads are in flight at once.  Every expression is
+// the march's, so the bits are the same.
+//
+// Registers, FP64: 124 (one row, 16 wavefronts a CU) and 158 (two rows, 12).  One
+// block runs per CU, so a step takes about 3 us of launch and loop control, one
+// memory round trip and the issue of the block's rows on four SIMDs (one row alone
+// 1.5 us, 20 rows 9 us).  Step time, the march at its best tile -> the block kernel:
+// FP64 64x64 8.3 -> 5.6 us, 256x256 10.9 -> 8.1, 501x363 15.3 -> 12.2, 512x512 17.5 -> 14.3.
+template <int RS, class P, int K, bool LOOP>
+__global__ __launch_bounds__(block_max_waves(K) * kLanes, block_max_waves(K) / 4)
+void step_block_kernel(KParams kp, Grid in, Grid out, double dt_arg, StepCtl *ctl, int ph) {
+  using T = typename P::T;
+  const int W = (int)(blockDim.x / kLanes);
+  const int R = K * W - 4;
+  constexpr bool kBnd = P::kSharedRecip;  // FP64 comes in bounded kinds only
+  static_assert(!kBnd || (RS & kRiemannFloorSqrt) != 0, "bounded FP64 kinds only");
+  constexpr bool kMinmod = (RS & kSlopeMinmod) != 0;
+  using Row = T[4][kLanes];
+  extern __shared__ __align__(16) unsigned char lds[];
+  // primitives; then the y flux below each wavefront's first row
+  Row *rows = reinterpret_cast<Row *>(lds);
+  Row *faces = rows + K * W;  // upper face states of each wavefront's last row
+  // per row, 1: outside the checked conversion, 2: out of bounds
+  int *flags = reinterpret_cast<int *>(faces + W);
+  const int lane = threadIdx.x & (kLanes - 1);
+  const int w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  LoopWords words;
+  if constexpr (LOOP) words = loop_words(ctl, ph);
+  const SchemeT<T> &s = P::scheme(kp);
+  const int strip = blockIdx.x, nstrips = gridDim.x, seg = blockIdx.y, nsegs = gridDim.y;
+  const int col = kOutCols * strip + lane;
+  const int j_base = 2 + R * seg;
+  const int r0 = j_base - 2 + K * w;  // this wavefront's first row
+
+  bool flipx;
+  const int c0 = ghost_map(min(col, kp.nx + 3), kp.nx, kp.bcxmin, kp.bcxmax, flipx);
+  typename P::Cell uc[K];
+#pragma unroll
+  for (int k = 0; k < K; k++) {
+    bool flipy;
+    const int rr = ghost_map_uniform(min(r0 + k, kp.ny + 3), kp.ny, kp.bcymin, kp.bcymax, flipy);
+    uc[k] = P::template load_rc<true>(in, rr, (unsigned)c0 * P::kElem);
+    if (flipx) P::negate(uc[k], IU);
+    if (flipy) P::negate(uc[k], IV);
+  }
+  double dt = dt_arg;
+  if constexpr (LOOP) {
+    const LoopPos L = loop_resolve(kp, words.t, words.nstep, words.slot);
+    if (strip == 0 && seg == 0 && w == 0) loop_publish(ctl, ph, L, lane);
+    if (!L.active) return;  // the loop has ended: every wavefront leaves, nothing is stored
+    dt = L.dt;
+  }
+  const T dtdx = (T)(dt / kp.dx);
+  const T dtdy = (T)(dt / kp.dy);
+
+  Q4T<T> q[K];
+  [[maybe_unused]] double rinv[K];
+#pragma unroll
+  for (int k = 0; k < K; k++) {
+    if constexpr (kBnd) {
+      bool rok, slow = !wave_all(dtdx <= kBndDtd && dtdy <= kBndDtd);
+      const bool all = wave_all(P::template prim_shared<true>(kp, uc[k], q[k], rinv[k], rok));
+      if (!all) {  // uniform
+        P::prim_ieee(kp, uc[k], q[k]);
+        slow = slow || !wave_all(!out_of_bounds(q[k]));
+      }
+      if (lane == 0) flags[K * w + k] = (all ? 0 : 1) | (slow ? 2 : 0);
+    } else {
+      P::prim(kp, uc[k], q[k]);
+    }
+    for (int v = 0; v < 4; v++) rows[K * w + k][v][lane] = q[k].v[v];
+  }
+  __syncthreads();
+
+  // slopes, source terms and face states of rows j_base - 1 .. j_base + R
+  Q4T<T> fymin[K] = {}, fymax[K] = {}, fxmin[K] = {}, ql[K] = {};
+  [[maybe_unused]] bool slow = false;
+  if constexpr (kBnd) {
+    int f = 0;
+    for (int k = 0; k < K * W; k++) f |= flags[k];
+    slow = (__builtin_amdgcn_readfirstlane(f) & 2) != 0;
+  }
+#pragma unroll
+  for (int k = 0; k < K; k++) {
+    const int row = K * w + k;
+    if (row < 1 || row > R + 2) continue;  // uniform
+    Q4T<T> qpy, qmy, fxmax, dqX = {}, dqY = {};
+    for (int v = 0; v < 4; v++) {
+      qpy.v[v] = k + 1 < K ? q[k + 1 < K ? k + 1 : k].v[v] : rows[row + 1][v][lane];
+      qmy.v[v] = k > 0 ? q[k > 0 ? k - 1 : k].v[v] : rows[row - 1][v][lane];
+    }
+    const Q4T<T> qpx = shfl_dn1(q[k]), qmx = shfl_up1(q[k]);
+    auto trace = [&](auto half, const SourcesT<T> &src) {
+      constexpr bool kHalf = decltype(half)::value;
+      trace_face<kHalf>(s, q[k], dqY, src, dtdy, false, fymin[k]);
+      trace_face<kHalf>(s, q[k], dqY, src, dtdy, true, fymax[k]);
+      trace_face<kHalf>(s, q[k], dqX, src, dtdx, false, fxmin[k]);
+      trace_face<kHalf>(s, q[k], dqX, src, dtdx, true, fxmax);
+    };
+    bool checked = false;  // the checked forms hold for the three rows this row reads
+    if constexpr (kBnd)
+      checked = !slow && __builtin_amdgcn_readfirstlane(flags[row - 1] | flags[row] |
+                                                        flags[row + 1]) == 0;
+    if constexpr (kMinmod) {
+      if (checked)  // uniform
+        slopes_xy<true>(s.slope_type, q[k], qpx, qmx, qpy, qmy, dqX, dqY);
+      else
+        slopes_xy<false>(s.slope_type, q[k], qpx, qmx, qpy, qmy, dqX, dqY);
+    } else if (s.slope_type != T(0.0)) {  // uniform
+      slopes_xy<false>(s.slope_type, q[k], qpx, qmx, qpy, qmy, dqX, dqY);
+    }
+    if constexpr (kBnd) {
+      if (checked) {  // uniform
+        bool ok = true;
+        trace(std::true_type{}, trace_sources_shared<true>(s, q[k], dqX, dqY, rinv[k], true, ok));
+      } else {
+        trace(std::false_type{}, trace_sources(s, q[k], dqX, dqY));
+      }
+    } else {
+      trace(std::false_type{}, trace_sources(s, q[k], dqX, dqY));
+    }
+    ql[k] = shfl_up1(fxmax);
+  }
+  for (int v = 0; v < 4; v++) faces[w][v][lane] = fymax[K - 1].v[v];
+  __syncthreads();
+
+  // y fluxes through the lower faces of rows j_base .. j_base + R, x fluxes of the
+  // output rows (the row above them forms one it does not use)
+  Q4T<T> fya[K] = {}, fxa[K] = {};
+#pragma unroll
+  for (int k = 0; k < K; k++) {
+    const int row = K * w + k;
+    if (row < 2 || row > R + 2) continue;  // uniform
+    Q4T<T> qd;
+    for (int v = 0; v < 4; v++)
+      qd.v[v] = k > 0 ? fymax[k > 0 ? k - 1 : k].v[v] : faces[w - 1][v][lane];
+    bool fok = true;
+    T fy[4], fx[4];
+    riemann<RS, kBnd>(s, qd, fymin[k], IV, IU, fy, fok);
+    riemann<RS, kBnd>(s, ql[k], fxmin[k], IU, IV, fx, fok);
+    if constexpr (kBnd) {
+      if (!wave_all(fok) || slow) {  // uniform
+        riemann<RS>(s, qd, fymin[k], IV, IU, fy);
+        riemann<RS>(s, ql[k], fxmin[k], IU, IV, fx);
+      }
+    }
+    for (int v = 0; v < 4; v++) {
+      fya[k].v[v] = fy[v] * dtdy;
+      fxa[k].v[v] = fx[v] * dtdx;
+    }
+  }
+  for (int v = 0; v < 4; v++) rows[K * w][v][lane] = fya[0].v[v];
+  __syncthreads();
+
+  const bool col_in = lane >= 2 && lane < 2 + kOutCols;
+  const bool out_col = col_in && col <= kp.nx + 1;
+  const bool col_ghost = col < 2 || (col > kp.nx + 1 && col <= kp.nx + 3);
+  const bool owned = out_col || (strip == 0 && lane < 2) ||
+                     (strip == nstrips - 1 && col > kp.nx + 1 && col <= kp.nx + 3);
+  const int row_lo = seg == 0 ? 0 : j_base;
+  const int row_hi = seg == nsegs - 1 ? kp.ny + 3 : min(j_base + R - 1, kp.ny + 1);
+  T rate = T(0.0);
+#pragma unroll
+  for (int k = 0; k < K; k++) {
+    const int row = K * w + k, r = r0 + k;
+    if (row >= 2 && row <= R + 1) {  // uniform
+      Q4T<T> fyt;
+      for (int v = 0; v < 4; v++)
+        fyt.v[v] = k + 1 < K ? fya[k + 1 < K ? k + 1 : k].v[v] : rows[row + 1][v][lane];
+      const Q4T<T> fxr = shfl_dn1(fxa[k]);
+      const typename P::Cell unew = P::update(uc[k], fxa[k], fxr, fya[k], fyt);
+      if (out_col && r <= kp.ny + 1) {
+        P::template store_rc<true>(out, r, (unsigned)col * P::kElem, unew);
+        if constexpr (LOOP)
+          rate = Ops<T>::mx(rate,
+                            cell_rate<P, (RS & kRiemannFloorSqrt) != 0, false>(kp, unew));
+      }
+    }
+    // ghost cells of this row that the block owns, in both arrays
+    if (r >= row_lo && r <= row_hi) {  // uniform
+      if (owned && (col_ghost || r < 2 || r > kp.ny + 1)) {
+        P::template store_rc<true>(in, r, (unsigned)col * P::kElem, uc[k]);
+        P::template store_rc<true>(out, r, (unsigned)col * P::kElem, uc[k]);
+      }
+    }
+  }
+  if constexpr (LOOP) {
+    if (K * w + K > 2 && K * w <= R + 1) {
+      const int p1 = ph == 2 ? 0 : ph + 1;
+      const unsigned slot = ((seg * nstrips + strip) * W + w) % kRateSlots;
+      reduce_rate_wave(rate, &ctl->rate[p1][slot * kSlotStride]);
+    }
   }
 }
 
@@ -1448,11 +1694,15 @@ __device__ __forceinline__ void batch_step_wave(const BatchInst *__restrict__ in
       Grid gout = gin;
       gout.p = even ? bi.U2.p : bi.U.p;
       const int strip = w % bi.nstrips, seg = w / bi.nstrips;
+      auto start = [&](double &dt) -> bool {
+        dt = L.dt;
+        return true;
+      };
       if (interior_cols(kp, strip))
-        wmax = march<RS, P, true, O32, false, 1>(kp, gin, gout, L.dt, seg_rows, bi.nstrips,
+        wmax = march<RS, P, true, O32, false, 1>(kp, gin, gout, start, seg_rows, bi.nstrips,
                                               strip, seg, false);
       else
-        wmax = march<RS, P, true, O32, true, 1>(kp, gin, gout, L.dt, seg_rows, bi.nstrips,
+        wmax = march<RS, P, true, O32, true, 1>(kp, gin, gout, start, seg_rows, bi.nstrips,
                                              strip, seg, false);
       target = rate_slot(ctl, ph);
     }
@@ -1461,9 +1711,9 @@ __device__ __forceinline__ void batch_step_wave(const BatchInst *__restrict__ in
 }
 
 template <int RS, class P, bool O32>
-__global__ __launch_bounds__(kBlock) void step_batch_kernel(const BatchInst *__restrict__ insts,
-                                                            int ninst, StepCtl *ctls, int ph,
-                                                            int nwaves, int seg_rows) {
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(2)))
+void step_batch_kernel(const BatchInst *__restrict__ insts, int ninst, StepCtl *ctls, int ph,
+                       int nwaves, int seg_rows) {
   batch_step_wave<RS, P, O32>(insts, ninst, ctls, ph, nwaves, seg_rows);
 }
 
@@ -1526,22 +1776,9 @@ __device__ __forceinline__ LoopPos loop_pos_coherent(const KParams &kp, StepCtl 
   }
   const unsigned long long b =
       lane < kRateSlots ? ctl_read(&ctl->rate[ph][lane * kSlotStride]) : 0ull;
-  LoopPos L;
-  // readfirstlane returns an int: the halves are taken as unsigned, so that a
-  // low half with its top bit set is not sign-extended into the high half
-  const unsigned tlo = (unsigned)__builtin_amdgcn_readfirstlane((unsigned)w0);
-  const unsigned thi = (unsigned)__builtin_amdgcn_readfirstlane((unsigned)(w0 >> 32));
-  L.t = __longlong_as_double((long long)(((unsigned long long)thi << 32) | tlo));
-  L.nstep = (int)__builtin_amdgcn_readfirstlane((unsigned)w1);
-  L.active = L.t < kp.tEnd && L.nstep < kp.nStepmax;
-  const long long mb = __double_as_longlong(wave_max(__longlong_as_double((long long)b)));
-  const unsigned mlo = __builtin_amdgcn_readfirstlane((unsigned)mb);
-  const unsigned mhi = __builtin_amdgcn_readfirstlane((unsigned)(mb >> 32));
-  const double invdt = __longlong_as_double((long long)(((unsigned long long)mhi << 32) | mlo));
-  double dt = kp.cfl / invdt;
-  if (L.t + dt > kp.tEnd) dt = kp.tEnd - L.t;
-  L.dt = dt;
-  return L;
+  return loop_resolve(kp, lane_value(__longlong_as_double((long long)w0), 0),
+                      (int)__builtin_amdgcn_readfirstlane((unsigned)w1),
+                      __longlong_as_double((long long)b));
 }
 
 __device__ __forceinline__ void loop_publish_coherent(StepCtl *ctl, int ph, const LoopPos &L,
@@ -1635,11 +1872,15 @@ __device__ __forceinline__ void batch_persistent_loop(const BatchInst *__restric
       Grid gout = gin;
       gout.p = even ? bi.U2.p : bi.U.p;
       const int strip = w % bi.nstrips, seg = w / bi.nstrips;
+      auto start = [&](double &dt) -> bool {
+        dt = L.dt;
+        return true;
+      };
       if (interior_cols(kp, strip))
-        wmax = march<RS, P, true, O32, false, 1>(kp, gin, gout, L.dt, seg_rows, bi.nstrips,
+        wmax = march<RS, P, true, O32, false, 1>(kp, gin, gout, start, seg_rows, bi.nstrips,
                                                  strip, seg, false);
       else
-        wmax = march<RS, P, true, O32, true, 1>(kp, gin, gout, L.dt, seg_rows, bi.nstrips,
+        wmax = march<RS, P, true, O32, true, 1>(kp, gin, gout, start, seg_rows, bi.nstrips,
                                                 strip, seg, false);
       reduce_rate_wave(wmax, rate_slot(ctl, ph));
     }
@@ -1650,9 +1891,10 @@ __device__ __forceinline__ void batch_persistent_loop(const BatchInst *__restric
 }
 
 template <int RS, class P, bool O32>
-__global__ __launch_bounds__(kBlock) void step_batch_persistent_kernel(
-    const BatchInst *__restrict__ insts, StepCtl *ctls, int ph0, int steps, BatchQueue q,
-    BatchCounters *cnt, unsigned *done, int seg_rows, unsigned spin_limit) {
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(2)))
+void step_batch_persistent_kernel(const BatchInst *__restrict__ insts, StepCtl *ctls, int ph0,
+                                  int steps, BatchQueue q, BatchCounters *cnt, unsigned *done,
+                                  int seg_rows, unsigned spin_limit) {
   batch_persistent_loop<RS, P, O32>(insts, ctls, ph0, steps, q, cnt, done, seg_rows, spin_limit);
 }
 
@@ -1804,9 +2046,55 @@ void launch_fused_t(const KParams &kp, Grid in, Grid out, double dt, StepCtl *ct
   }
 }
 
+template <int RS, class P, int K>
+void launch_block_k(const KParams &kp, Grid in, Grid out, double dt, StepCtl *ctl, int ph,
+                    const BlockMap &m, hipStream_t st) {
+  const dim3 grid((unsigned)m.nstrips, (unsigned)m.nsegs), block(m.waves * kLanes);
+  const size_t lds =
+      (size_t)(K + 1) * m.waves * 4 * kLanes * sizeof(typename P::T) + K * m.waves * sizeof(int);
+  if (ctl)
+    hipLaunchKernelGGL((step_block_kernel<RS, P, K, true>), grid, block, lds, st, kp, in, out, dt,
+                       ctl, ph);
+  else
+    hipLaunchKernelGGL((step_block_kernel<RS, P, K, false>), grid, block, lds, st, kp, in, out, dt,
+                       ctl, ph);
+}
+
+template <int RS, class P>
+void launch_block_rs(const KParams &kp, Grid in, Grid out, double dt, StepCtl *ctl, int ph,
+                     const BlockMap &m, hipStream_t st) {
+  if (m.k == 1)
+    launch_block_k<RS, P, 1>(kp, in, out, dt, ctl, ph, m, st);
+  else
+    launch_block_k<RS, P, 2>(kp, in, out, dt, ctl, ph, m, st);
+}
+
+template <class P>
+void launch_block(const KParams &kp, Grid in, Grid out, double dt, StepCtl *ctl, int ph,
+                  const BlockMap &m, hipStream_t st) {
+  const bool c = kp.s.riemann == 2;  // HLLC; else HLL
+  if constexpr (std::is_same<P, P64>::value) {
+    constexpr int fs = kRiemannFloorSqrt;
+    if (kp.s.slope_type == 1.0)
+      c ? launch_block_rs<2 | fs | kSlopeMinmod, P>(kp, in, out, dt, ctl, ph, m, st)
+        : launch_block_rs<1 | fs | kSlopeMinmod, P>(kp, in, out, dt, ctl, ph, m, st);
+    else
+      c ? launch_block_rs<2 | fs, P>(kp, in, out, dt, ctl, ph, m, st)
+        : launch_block_rs<1 | fs, P>(kp, in, out, dt, ctl, ph, m, st);
+  } else {
+    c ? launch_block_rs<2, P>(kp, in, out, dt, ctl, ph, m, st)
+      : launch_block_rs<1, P>(kp, in, out, dt, ctl, ph, m, st);
+  }
+}
+
 template <class P>
 void launch_fused_p(const KParams &kp, Grid in, Grid out, double dt, StepCtl *ctl, int ph,
                     int seg_rows, hipStream_t st) {
+  const BlockMap m = block_map(kp, seg_rows);
+  if (m.k > 0 && off32_ok(kp, in) && off32_ok(kp, out)) {
+    launch_block<P>(kp, in, out, dt, ctl, ph, m, st);
+    return;
+  }
   if constexpr (std::is_same<P, P64>::value) {
     if (kp.s.floor_sqrt && kp.s.riemann != 0) {  // HLL / HLLC with the short square root
       // minmod slopes and power-of-two cell sizes built in: run-loop launches
@@ -2043,6 +2331,48 @@ hipError_t launch_step_fused(const KParams &kp, Grid in, Grid out, double dt, St
   else
     launch_fused_p<P64>(kp, in, out, dt, ctl, ph, seg_rows, st);
   return hipGetLastError();
+}
+
+BlockMap block_map(const KParams &kp, int seg_rows) {
+  BlockMap m{};
+  if (seg_rows > 2 * block_max_waves(2) - 4) return m;
+  // built for HLL and HLLC, in FP64 for the bounded kinds
+  if (kp.s.riemann == 0 || (kp.prec == E2D_PRECISION_FP64 && !kp.s.floor_sqrt)) return m;
+  const int k = seg_rows <= block_max_waves(1) - 4 ? 1 : 2;
+  m.waves = (seg_rows + 4 + k - 1) / k;
+  const int rows = k * m.waves - 4;
+  m.nstrips = (kp.nx + kOutCols - 1) / kOutCols;
+  m.nsegs = (kp.ny + rows - 1) / rows;
+  // one block per CU: past that a second round of blocks costs a whole step again
+  // (512x512, 8 rows, 576 blocks: 19.8 us; 20 rows, 234 blocks: 14.1; the
+  // march's best 16.6)
+  if ((long long)m.nstrips * m.nsegs <= kp.simds / 4) m.k = k;
+  return m;
+}
+
+double march_cost(double waves, int tile, int simds) {
+  const double n = waves / (simds > 0 ? simds : 1024);  // wavefronts per SIMD
+  const double rows = tile + 2.0;
+  // many rounds of wavefronts: the chip stays full until the last ones march
+  if (n > 8.0) return n * rows + 0.6 * rows;
+  // few: pairs that share a SIMD, then what is left of a pair
+  const double pairs = std::floor(n / 2.0), rest = n - 2.0 * pairs;
+  return 2.0 * pairs * rows + (rest <= 0.0 ? 0.0 : rest <= 1.0 ? 1.35 * rows : 2.0 * rows);
+}
+
+int auto_tile(const KParams &kp) {
+  for (int tile = 1; tile <= 2 * block_max_waves(2) - 4; ++tile)
+    if (block_map(kp, tile).k > 0) return tile;
+  int best = 16;
+  double least = 1e300;
+  for (int tile = 3; tile <= 96; ++tile) {
+    const double c = march_cost(fused_map(kp, tile).nwaves, tile, kp.simds);
+    if (c < least) {
+      least = c;
+      best = tile;
+    }
+  }
+  return best;
 }
 
 FusedMap fused_map(const KParams &kp, int seg_rows) {

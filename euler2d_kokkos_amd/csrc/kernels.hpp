@@ -147,6 +147,31 @@ struct FusedMap {
 };
 FusedMap fused_map(const KParams &kp, int seg_rows);
 
+// Work map of the block step kernel: one block of `waves` wavefronts, each with
+// k loaded rows, per segment of k * waves - 4 output rows of a strip.  k = 0:
+// this tile runs the march.
+struct BlockMap {
+  int k, waves;
+  int nstrips, nsegs;
+};
+// wavefronts of the largest block: as many as a CU holds at the kernel's registers
+constexpr int block_max_waves(int k) { return k == 1 ? 16 : 12; }
+// A tile runs the block kernel where its blocks fit one per CU of the device.
+BlockMap block_map(const KParams &kp, int seg_rows);
+
+// Relative time of a step whose `waves` wavefronts march `tile` rows each (plus
+// warm-up rows worth two) on `simds` SIMDs that hold two at a time: two that
+// share a SIMD take 2 units a row, one alone 1.35.  Against measured times: FP64
+// 1024x1536, tiles 7 / 10 / 12 / 14 / 16 / 20: 36 / 38 / 47 / 32 / 36 / 44 units,
+// 51.0 / 52.8 / 59.2 / 43.6 / 49.5 / 55.8 us; 3001x1777, tiles 14 / 24 / 48: 118 / 104 / 100
+// units, 160 / 154 / 144 us.
+double march_cost(double waves, int tile, int simds);
+// The tile a run starts with: the smallest whose blocks fit one per CU (a
+// smaller one shortens each wavefront's chain as long as no second round of
+// blocks is needed: 256x256, tiles 6 / 8 / 12: 8.1 / 8.5 / 10.1 us); for larger
+// grids the march's tile of least march_cost.
+int auto_tile(const KParams &kp);
+
 KParams make_kparams(const e2d_params &p, int precision);
 // planes of one state array (one per conserved variable) and bytes of one
 // element: a double (FP64), a (hi, lo) pair of floats (split) or a float
