@@ -90,7 +90,7 @@ struct e2d_run {
   e2d::KParams kp{};
   int precision = 0;
   int schedule = E2D_SCHEDULE_FUSED;
-  int seg_rows = 16;
+  int seg_rows = 16;  // e2d_create chooses it from the grid
   int device = 0;
   hipStream_t stream = nullptr;
   Grid U{}, U2{}, Q{}, Fx{}, Fy{}, Sx{}, Sy{};
@@ -735,6 +735,7 @@ int e2d_create(const e2d_params *p, int precision, e2d_run **out) {
     int ncu = 0;
     HIP_TRY(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, r->device));
     r->kp.simds = 4 * ncu;
+    r->seg_rows = e2d::auto_tile(r->kp);
     HIP_TRY(hipStreamCreateWithFlags(&r->stream, hipStreamNonBlocking));
     void *ptr = nullptr;
     int rc2 = alloc_grid(r, r->U, precision);
@@ -1020,6 +1021,9 @@ int e2d_autotune(e2d_run *r, const int *candidates, int ncand, int steps, int *b
     // tiles at which the step's wavefronts fit k per SIMD (k = 1..4) are the
     // natural candidates, next to a fixed set.
     auto_cand = {8, 12, 14, 16, 20, 24, 32, 48, 64};
+    const int first = e2d::auto_tile(r->kp);
+    if (std::find(auto_cand.begin(), auto_cand.end(), first) == auto_cand.end())
+      auto_cand.push_back(first);
     hipDeviceProp_t prop;
     if (hipGetDeviceProperties(&prop, r->device) == hipSuccess) {
       const int simds = 4 * prop.multiProcessorCount;
@@ -1134,6 +1138,7 @@ struct e2d_batch {
   double queue_imbalance = 1.0;          // cells of the fullest XCD queue / the mean
   long long max_items = (1LL << 31) - 1;  // work items of one persistent launch, at most
   bool launch_chosen = false;            // e2d_batch_set_launch has fixed the mode
+  bool tile_chosen = false;              // e2d_batch_set_tile or the autotuner has fixed the tile
   unsigned spin_limit = 0;
   int nxcd = 0;                          // XCDs seen by the probe at creation
   int xmap[e2d::kMaxXcds];               // XCC id -> queue (-1: not seen)
@@ -1171,9 +1176,14 @@ void batch_drop_graph(e2d_batch *b) {
 // of about 64 cycles, about a second in all
 constexpr unsigned kDefaultSpinLimit = 1u << 20;
 
-// largest queue imbalance (fullest XCD queue's cells over the mean) at which
-// a new batch defaults to the persistent launch
+// A new batch defaults to the persistent launch where its instances fill the XCD
+// queues evenly (fullest queue's cells over the mean) and each queue holds enough
+// of them that a wavefront hardly ever waits for its instance's previous step.
+// us per step, one launch per step / persistent, best tiles: 48 instances (6 a
+// queue, 2.7 Mcell) FP64 94 / 103, split 56 / 78; 96 (12 a queue) 185 / 177, 122 / 116;
+// 192: 333 / 316, 226 / 218.
 constexpr double kPersistentImbalance = 1.10;
+constexpr int kPersistentPerQueue = 12;
 
 // Work queues of the persistent launch for the current tile: instances go to
 // the XCD with the least work so far, largest first (cells as the measure);
@@ -1254,6 +1264,42 @@ int batch_upload_table(e2d_batch *b) {
   HIP_TRY(hipStreamSynchronize(b->stream));
   batch_drop_graph(b);
   return E2D_OK;
+}
+
+int batch_tile(e2d_batch *b, int seg_rows) {
+  b->seg_rows = seg_rows;
+  return batch_upload_table(b);
+}
+
+// The tile of the current launch mode while the caller has chosen none.  One
+// launch per step: the march's least cost over all instances.  Persistent: no tail per
+// step, so FP64 takes longer segments, about 3.5 wavefronts per SIMD (192 instances,
+// tiles 14 / 32 / 64: 356 / 327 / 316 us), while split precision wants its third
+// wavefront per SIMD (prefetch distance 1, short segments; tiles 14 / 20 / 48: 229 /
+// 218 / 222 us).
+int batch_auto_tile(const e2d_batch *b) {
+  auto waves = [&](int tile) {
+    long long w = 0;
+    for (const e2d_run *r : b->runs) w += e2d::batch_waves(r->kp, tile, nullptr);
+    return (double)w;
+  };
+  const int simds = b->runs[0]->kp.simds;
+  if (b->launch == E2D_BATCH_LAUNCH_PERSISTENT) {
+    if (b->precision != E2D_PRECISION_FP64) return 20;
+    int tile = 16;
+    while (tile < 64 && waves(tile) > 3.5 * simds) tile += 4;
+    return tile;
+  }
+  int best = 14;
+  double least = 1e300;
+  for (int tile = 4; tile <= 64; ++tile) {
+    const double c = e2d::march_cost(waves(tile), tile, simds);
+    if (c < least) {
+      least = c;
+      best = tile;
+    }
+  }
+  return best;
 }
 
 int batch_launch(e2d_batch *b) {
@@ -1389,7 +1435,7 @@ int e2d_batch_set_launch(e2d_batch *b, int mode, int spin_limit) {
   b->launch = mode;
   b->launch_chosen = true;
   b->spin_limit = spin_limit > 0 ? (unsigned)spin_limit : 0u;
-  return E2D_OK;
+  return guarded([&]() -> int { return b->tile_chosen ? E2D_OK : batch_tile(b, batch_auto_tile(b)); });
 }
 
 int e2d_batch_get_launch(e2d_batch *b, int *mode) {
@@ -1499,10 +1545,17 @@ int e2d_batch_create(const e2d_params *params, int count, int precision, e2d_bat
       if (v > 0 && v < b->max_items) b->max_items = v;
     }
     // The persistent launch keeps each instance on one XCD: it is the default
-    // when the instances fill the XCD queues evenly, and one launch per step
+    // when the instances fill the XCD queues well, and one launch per step
     // (every instance over the whole GPU) otherwise, e.g. for a few large grids.
-    b->launch = b->queue_imbalance <= kPersistentImbalance ? E2D_BATCH_LAUNCH_PERSISTENT
-                                                           : E2D_BATCH_LAUNCH_STEPS;
+    b->launch = b->queue_imbalance <= kPersistentImbalance && count >= kPersistentPerQueue * b->nxcd
+                    ? E2D_BATCH_LAUNCH_PERSISTENT
+                    : E2D_BATCH_LAUNCH_STEPS;
+    rc = batch_tile(b, batch_auto_tile(b));
+    if (rc) {
+      const std::string msg = g_last_error;
+      e2d_batch_destroy(b);
+      return fail(rc, msg);
+    }
     *out = b;
     return E2D_OK;
   });
@@ -1550,8 +1603,8 @@ int e2d_batch_set_tile(e2d_batch *b, int seg_rows) {
   int rc = batch_check(b);
   if (rc) return rc;
   if (seg_rows < 1 || seg_rows > 4096) return fail(E2D_ERR_ARG, "seg_rows must be in [1, 4096]");
-  b->seg_rows = seg_rows;
-  return batch_upload_table(b);
+  b->tile_chosen = true;
+  return batch_tile(b, seg_rows);
 }
 
 int e2d_batch_run(e2d_batch *b, int max_steps, int use_graph, double *elapsed_ms,

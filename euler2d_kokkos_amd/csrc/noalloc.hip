@@ -106,7 +106,7 @@ extern "C" int e2d_run_loop_noalloc(const e2d_params *p, int precision, void *U,
   kp.wide_addr = (unsigned long long)plane * (unsigned long long)esize > (1ull << 32);
   const Grid gU{U, (int)pitch, plane};
   const Grid gU2{U2, (int)pitch, plane};
-  const int tile = seg_rows > 0 ? seg_rows : 16;
+  const int tile = seg_rows > 0 ? seg_rows : e2d::auto_tile(kp);
   hipStream_t st = static_cast<hipStream_t>(stream);
 
   // loop start: arrival counter cleared, then the CFL rate of the step's input

@@ -204,7 +204,8 @@ int e2d_run_loop(e2d_run *run, int max_steps, double *t, int *nStep);
  *             (FP32); aligned to the element size
  *   pitch     elements between rows (>= isize); plane: elements between
  *             planes (>= pitch * jsize)
- *   seg_rows  the step kernel's tile (0: 16; results do not depend on it)
+ *   seg_rows  the step kernel's tile (0: chosen from the grid, as e2d_create
+ *             does; results do not depend on it)
  *   stream    a hipStream_t (NULL: the default stream)
  * Otherwise as e2d_run_loop: *t and *nStep hold the loop state on entry and
  * on return; at *nStep == 0 the ghost cells of both arrays are filled first;
@@ -236,8 +237,10 @@ int e2d_kinetic_cells(e2d_run *run, int which, long long *count);
  * 1 -> DIRECTIONAL, 2 -> ATOMIC.  Every schedule but FUSED is FP64 only. */
 int e2d_set_schedule(e2d_run *run, int schedule);
 int e2d_get_schedule(e2d_run *run, int *schedule);
-/* rows marched by one wavefront of the fused step kernel (1..4096); the
- * wavefront covers 60 output columns.  Results do not depend on it. */
+/* Output rows of one work item of the fused step (1..4096), 60 columns wide: the
+ * rows that one wavefront marches, or, where the items fit one per CU (small
+ * grids, up to 20 rows), the rows of one block of wavefronts.  e2d_create
+ * chooses it from the grid.  Results do not depend on it. */
 int e2d_set_tile(e2d_run *run, int seg_rows);
 int e2d_get_tile(e2d_run *run, int *seg_rows);
 /* Times `steps` loop iterations for each candidate seg_rows on the current
@@ -311,8 +314,9 @@ int e2d_batch_set_tile(e2d_batch *batch, int seg_rows);
  *                                replayed from hipGraphs when use_graph != 0
  * A new batch takes the persistent launch when its instances fill the XCD
  * queues evenly (the fullest queue holds at most 10% more cells than the
- * mean), else one launch per step (a few large grids would otherwise leave
- * XCDs idle); e2d_batch_get_launch reports the choice.
+ * mean) and there are at least 12 per queue, else one launch per step (fewer
+ * grids would leave wavefronts waiting or XCDs idle); e2d_batch_get_launch
+ * reports the choice.  Until e2d_batch_set_tile, the tile follows the mode.
  * spin_limit bounds each dependency wait of the persistent launch (polls of
  * the completion count, each about a microsecond; <= 0: the default, 2^20,
  * about a second); a wait that runs past it ends
