@@ -85,6 +85,8 @@ struct Staging {
   hipEvent_t ev[8] = {};
 };
 
+constexpr int kStepEvents = 32;
+
 struct e2d_run {
   e2d_params p{};
   e2d::KParams kp{};
@@ -96,7 +98,12 @@ struct e2d_run {
   Grid U{}, U2{}, Q{}, Fx{}, Fy{}, Sx{}, Sy{};
   e2d::StepCtl *ctl = nullptr;
   e2d::StepState *host_s = nullptr;  // pinned copy of ctl->s, written by the step kernels
+  double *host_rate = nullptr;       // pinned word behind host_s, for e2d_compute_dt
   hipEvent_t ev0 = nullptr, ev1 = nullptr;  // the run loop's timing events
+  // events around the fused steps of e2d_godunov_unsplit that the timers have
+  // not counted yet (steps step_done .. step_next - 1, each in slot k % kStepEvents)
+  hipEvent_t step_ev[kStepEvents][2] = {};
+  long long step_done = 0, step_next = 0;
   int phase = 0;  // phase of the next run-loop launch in the control rings
   // captured runs of kLoopGraphSteps[g] run-loop launches (for seg_rows = loop_graph_tile[g])
   hipGraphExec_t loop_graph[2] = {nullptr, nullptr};
@@ -182,83 +189,102 @@ int ensure_pass_arrays(e2d_run *r) {
   return rc;
 }
 
+// Adds the device time of the fused steps up to number `upto` to the timers.
+int count_steps(e2d_run *r, long long upto) {
+  for (; r->step_done < upto; ++r->step_done) {
+    hipEvent_t *ev = r->step_ev[r->step_done % kStepEvents];
+    HIP_TRY(hipEventSynchronize(ev[1]));
+    float ms = 0.f;
+    HIP_TRY(hipEventElapsedTime(&ms, ev[0], ev[1]));
+    r->timers[1] += ms * 1e-3;
+  }
+  return E2D_OK;
+}
+
+// One fused step with an explicit dt, queued with events of its own: the host
+// neither waits for the step nor makes events for it (together 30 us a call at
+// 512x512, more than the step).  The timers are brought up to date when they are
+// read, or when an event's slot comes round again.
+int queue_step(e2d_run *r, const Grid &in, const Grid &out, double dt) {
+  int rc = count_steps(r, r->step_next - kStepEvents + 1);
+  if (rc) return rc;
+  hipEvent_t *ev = r->step_ev[r->step_next % kStepEvents];
+  for (int k = 0; k < 2; ++k)
+    if (!ev[k]) HIP_TRY(hipEventCreate(&ev[k]));
+  HIP_TRY(hipEventRecord(ev[0], r->stream));
+  // implementation version 0 as one fused launch (boundaries to update)
+  e2d::Region impl("hydro_impl0");
+  HIP_TRY(e2d::launch_step_fused(r->kp, in, out, dt, nullptr, 0, r->seg_rows, r->stream));
+  HIP_TRY(hipEventRecord(ev[1], r->stream));
+  ++r->step_next;
+  return E2D_OK;
+}
+
 // one godunov step with an explicit dt; in/out by the parity of nStep
 int do_step(e2d_run *r, int nStep, double dt, bool timed) {
   Grid in = (nStep % 2 == 0) ? r->U : r->U2;
   Grid out = (nStep % 2 == 0) ? r->U2 : r->U;
+  if (r->schedule == E2D_SCHEDULE_FUSED) return queue_step(r, in, out, dt);
   const double dtdx = dt / r->p.dx;
   const double dtdy = dt / r->p.dy;
   Events<5> evs;
   hipEvent_t *ev = evs.e;
   if (timed) HIP_TRY(evs.create());
-  if (r->schedule != E2D_SCHEDULE_FUSED) {
-    if (r->precision != E2D_PRECISION_FP64)
-      return fail(E2D_ERR_UNSUPPORTED, "the pass schedules exist for FP64 only");
-    int rc = ensure_pass_arrays(r);
-    if (rc) return rc;
-    // HydroRun::godunov_unsplit_impl, HydroRun.h:279-364
-    if (timed) HIP_TRY(hipEventRecord(ev[0], r->stream));
-    {
-      e2d::Region reg("make_boundaries");
-      HIP_TRY(e2d::launch_boundaries(r->kp, in, r->stream));
-    }
-    HIP_TRY(e2d::launch_copy(r->kp, in, out, r->stream));
-    if (timed) HIP_TRY(hipEventRecord(ev[1], r->stream));
-    {
-      e2d::Region reg("compute_primitives");
-      HIP_TRY(e2d::launch_prim(r->kp, in, r->Q, r->stream));
-    }
-    if (timed) HIP_TRY(hipEventRecord(ev[2], r->stream));
-    if (r->schedule == E2D_SCHEDULE_PASSES) {
-      e2d::Region impl("hydro_impl0");
-      {
-        e2d::Region reg("compute_fluxes");
-        HIP_TRY(e2d::launch_fluxes(r->kp, r->Q, r->Fx, r->Fy, dtdx, dtdy, r->stream));
-      }
-      if (timed) HIP_TRY(hipEventRecord(ev[3], r->stream));
-      e2d::Region reg("update_hydro");
-      HIP_TRY(e2d::launch_update(r->kp, out, r->Fx, r->Fy, r->stream));
-    } else if (r->schedule == E2D_SCHEDULE_DIRECTIONAL) {
-      e2d::Region impl("hydro_impl1");
-      HIP_TRY(e2d::launch_slopes(r->kp, r->Q, r->Sx, r->Sy, r->stream));
-      HIP_TRY(e2d::launch_trace_fluxes(r->kp, 0, r->Q, r->Sx, r->Sy, r->Fx, dtdx, dtdy,
-                                       r->stream));
-      HIP_TRY(e2d::launch_update_dir(r->kp, 0, out, r->Fx, r->stream));
-      HIP_TRY(e2d::launch_trace_fluxes(r->kp, 1, r->Q, r->Sx, r->Sy, r->Fy, dtdx, dtdy,
-                                       r->stream));
-      HIP_TRY(e2d::launch_update_dir(r->kp, 1, out, r->Fy, r->stream));
-    } else {
-      e2d::Region impl("hydro_impl2");
-      HIP_TRY(e2d::launch_fluxes_atomic(r->kp, r->Q, out, dtdx, dtdy, r->stream));
-    }
-    if (timed) HIP_TRY(hipEventRecord(ev[4], r->stream));
-  } else {
-    if (timed) HIP_TRY(hipEventRecord(ev[0], r->stream));
-    // implementation version 0 as one fused launch (boundaries to update)
-    e2d::Region impl("hydro_impl0");
-    HIP_TRY(e2d::launch_step_fused(r->kp, in, out, dt, nullptr, 0, r->seg_rows, r->stream));
-    if (timed) HIP_TRY(hipEventRecord(ev[4], r->stream));
+  if (r->precision != E2D_PRECISION_FP64)
+    return fail(E2D_ERR_UNSUPPORTED, "the pass schedules exist for FP64 only");
+  int rc = ensure_pass_arrays(r);
+  if (rc) return rc;
+  // HydroRun::godunov_unsplit_impl, HydroRun.h:279-364
+  if (timed) HIP_TRY(hipEventRecord(ev[0], r->stream));
+  {
+    e2d::Region reg("make_boundaries");
+    HIP_TRY(e2d::launch_boundaries(r->kp, in, r->stream));
   }
+  HIP_TRY(e2d::launch_copy(r->kp, in, out, r->stream));
+  if (timed) HIP_TRY(hipEventRecord(ev[1], r->stream));
+  {
+    e2d::Region reg("compute_primitives");
+    HIP_TRY(e2d::launch_prim(r->kp, in, r->Q, r->stream));
+  }
+  if (timed) HIP_TRY(hipEventRecord(ev[2], r->stream));
+  if (r->schedule == E2D_SCHEDULE_PASSES) {
+    e2d::Region impl("hydro_impl0");
+    {
+      e2d::Region reg("compute_fluxes");
+      HIP_TRY(e2d::launch_fluxes(r->kp, r->Q, r->Fx, r->Fy, dtdx, dtdy, r->stream));
+    }
+    if (timed) HIP_TRY(hipEventRecord(ev[3], r->stream));
+    e2d::Region reg("update_hydro");
+    HIP_TRY(e2d::launch_update(r->kp, out, r->Fx, r->Fy, r->stream));
+  } else if (r->schedule == E2D_SCHEDULE_DIRECTIONAL) {
+    e2d::Region impl("hydro_impl1");
+    HIP_TRY(e2d::launch_slopes(r->kp, r->Q, r->Sx, r->Sy, r->stream));
+    HIP_TRY(e2d::launch_trace_fluxes(r->kp, 0, r->Q, r->Sx, r->Sy, r->Fx, dtdx, dtdy,
+                                     r->stream));
+    HIP_TRY(e2d::launch_update_dir(r->kp, 0, out, r->Fx, r->stream));
+    HIP_TRY(e2d::launch_trace_fluxes(r->kp, 1, r->Q, r->Sx, r->Sy, r->Fy, dtdx, dtdy,
+                                     r->stream));
+    HIP_TRY(e2d::launch_update_dir(r->kp, 1, out, r->Fy, r->stream));
+  } else {
+    e2d::Region impl("hydro_impl2");
+    HIP_TRY(e2d::launch_fluxes_atomic(r->kp, r->Q, out, dtdx, dtdy, r->stream));
+  }
+  if (timed) HIP_TRY(hipEventRecord(ev[4], r->stream));
   if (timed) {
     HIP_TRY(hipEventSynchronize(ev[4]));
     float ms = 0.f;
-    if (r->schedule != E2D_SCHEDULE_FUSED) {
-      HIP_TRY(hipEventElapsedTime(&ms, ev[0], ev[1]));
-      r->timers[0] += ms * 1e-3;
-      HIP_TRY(hipEventElapsedTime(&ms, ev[1], ev[2]));
-      r->timers[2] += ms * 1e-3;
-      if (r->schedule == E2D_SCHEDULE_PASSES) {  // flux / update timers of version 0 only
-        HIP_TRY(hipEventElapsedTime(&ms, ev[2], ev[3]));
-        r->timers[3] += ms * 1e-3;
-        HIP_TRY(hipEventElapsedTime(&ms, ev[3], ev[4]));
-        r->timers[4] += ms * 1e-3;
-      }
-      HIP_TRY(hipEventElapsedTime(&ms, ev[1], ev[4]));
-      r->timers[1] += ms * 1e-3;
-    } else {
-      HIP_TRY(hipEventElapsedTime(&ms, ev[0], ev[4]));
-      r->timers[1] += ms * 1e-3;
+    HIP_TRY(hipEventElapsedTime(&ms, ev[0], ev[1]));
+    r->timers[0] += ms * 1e-3;
+    HIP_TRY(hipEventElapsedTime(&ms, ev[1], ev[2]));
+    r->timers[2] += ms * 1e-3;
+    if (r->schedule == E2D_SCHEDULE_PASSES) {  // flux / update timers of version 0 only
+      HIP_TRY(hipEventElapsedTime(&ms, ev[2], ev[3]));
+      r->timers[3] += ms * 1e-3;
+      HIP_TRY(hipEventElapsedTime(&ms, ev[3], ev[4]));
+      r->timers[4] += ms * 1e-3;
     }
+    HIP_TRY(hipEventElapsedTime(&ms, ev[1], ev[4]));
+    r->timers[1] += ms * 1e-3;
   }
   return E2D_OK;
 }
@@ -753,9 +779,11 @@ int e2d_create(const e2d_params *p, int precision, e2d_run **out) {
     if (rc2) return rc2;
     HIP_TRY(hipEventCreate(&r->ev0));
     HIP_TRY(hipEventCreate(&r->ev1));
-    HIP_TRY(hipHostMalloc(reinterpret_cast<void **>(&r->host_s), 3 * sizeof(e2d::StepState),
+    const size_t host_bytes = 3 * sizeof(e2d::StepState) + sizeof(double);
+    HIP_TRY(hipHostMalloc(reinterpret_cast<void **>(&r->host_s), host_bytes,
                           hipHostMallocDefault));
-    std::memset(r->host_s, 0, 3 * sizeof(e2d::StepState));
+    std::memset(r->host_s, 0, host_bytes);
+    r->host_rate = reinterpret_cast<double *>(r->host_s + 3);
     // 32-bit row offsets in the step kernels need planes of at most 4 GiB;
     // E2D_WIDE_ADDRESSING=1 selects the 64-bit form for any size
     const char *wide = std::getenv("E2D_WIDE_ADDRESSING");
@@ -789,6 +817,9 @@ int e2d_destroy(e2d_run *run) {
   if (run->stream) (void)hipStreamSynchronize(run->stream);
   for (hipGraphExec_t g : run->loop_graph)
     if (g) (void)hipGraphExecDestroy(g);
+  for (auto &pair : run->step_ev)
+    for (hipEvent_t e : pair)
+      if (e) (void)hipEventDestroy(e);
   if (run->ev0) (void)hipEventDestroy(run->ev0);
   if (run->ev1) (void)hipEventDestroy(run->ev1);
   if (run->host_s) (void)hipHostFree(run->host_s);
@@ -835,14 +866,12 @@ int e2d_compute_dt(e2d_run *r, int useU, double *dt) {
   if (rc) return rc;
   if (!dt) return fail(E2D_ERR_ARG, "null dt");
   e2d::Region reg("compute_dt");
-  HIP_TRY(hipMemsetAsync(r->bits, 0, sizeof(unsigned long long), r->stream));
-  HIP_TRY(e2d::launch_dt_reduce(r->kp, useU == 0 ? r->U : r->U2, r->bits, r->stream));
-  unsigned long long bits = 0;
-  HIP_TRY(hipMemcpyAsync(&bits, r->bits, sizeof(bits), hipMemcpyDeviceToHost, r->stream));
+  // one launch, whose last block leaves the rate in pinned host memory
+  const Grid &g = useU == 0 ? r->U : r->U2;
+  HIP_TRY(e2d::launch_loop_begin(r->kp, g, g, 0, r->ctl, 0.0, 0, r->partials, r->stream,
+                                 r->host_rate));
   HIP_TRY(hipStreamSynchronize(r->stream));
-  double invdt;
-  std::memcpy(&invdt, &bits, sizeof(invdt));
-  *dt = r->p.cfl / invdt;  // HydroRun.h:246
+  *dt = r->p.cfl / *(const volatile double *)r->host_rate;  // HydroRun.h:246
   return E2D_OK;
 }
 
@@ -978,6 +1007,11 @@ int e2d_radial_profile(e2d_run *r, int which, int nbins, double *distances, doub
 
 int e2d_timers(e2d_run *r, double out[5]) {
   if (!r || !out) return fail(E2D_ERR_ARG, "null argument");
+  if (r->step_done < r->step_next) {
+    int rc = check_run(r);
+    if (!rc) rc = count_steps(r, r->step_next);
+    if (rc) return rc;
+  }
   for (int k = 0; k < 5; k++) out[k] = r->timers[k];
   return E2D_OK;
 }

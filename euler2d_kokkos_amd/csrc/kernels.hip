@@ -609,23 +609,32 @@ __device__ __forceinline__ void mirror_state(StepState *hs, int ph, const StepSt
 }
 
 // Start of a run loop in one launch (main.cpp:90-91 and the first compute_dt,
-// HydroRun.h:227-251): block b folds the CFL rate of interior rows b, b + G,
-// ... into partials[b]; with `bc` the grid's threads also fill the ghost cells
-// of `in` and `other` (make_boundaries of both arrays before step 0: the ghost
-// cells written are disjoint from the interior cells read).  The last block
-// to arrive (atomicInc wraps the arrival counter back to 0 for the next use)
-// takes the max of the partials and sets ring phase 0: the state before the
-// step and its rate in s[0] / rate[0], rate[1] cleared for launch 0's fold.
-// Launch 0 clears rate[2] itself.  Blocks of 16 wavefronts keep the loads of
-// many rows in flight (with 4 the kernel waited on load latency).
+// HydroRun.h:227-251): the wavefronts fold the CFL rate of the interior cells,
+// 64 columns x 4 rows at a time, and each block stores its maximum in partials;
+// with `bc` the grid's threads also fill the ghost cells of `in` and `other`
+// (make_boundaries of both arrays before step 0: the ghost cells written are
+// disjoint from the interior cells read).  The last block to arrive (atomicInc
+// wraps the arrival counter back to 0 for the next use) takes the max of the
+// partials and sets ring phase 0: the state before the step and its rate in s[0] /
+// rate[0], rate[1] cleared for launch 0's fold.  Launch 0 clears rate[2] itself.
+// With host_rate the maximum goes there instead (pinned host memory; e2d_compute_dt).
+// Blocks of 16 wavefronts keep the loads of many rows in flight (with 4 the kernel
+// waited on load latency); as many blocks as give each wavefront one piece, at
+// most kBeginBlocks: a small grid waits for few arrivals (one block at 64x64).
 constexpr int kBeginThreads = 1024;
+constexpr int kBeginRows = 4;
+
+int begin_blocks(const KParams &kp) {
+  const long long pieces = (long long)((kp.nx + kLanes - 1) / kLanes) *
+                           ((kp.ny + kBeginRows - 1) / kBeginRows);
+  const int waves = kBeginThreads / kLanes;
+  return (int)std::min<long long>(kBeginBlocks, (pieces + waves - 1) / waves);
+}
 
 template <class P>
-__global__ __launch_bounds__(kBeginThreads) void loop_begin_kernel(KParams kp, Grid in,
-                                                                   Grid other, int bc,
-                                                                   StepCtl *ctl, double t,
-                                                                   int nstep, double *partials,
-                                                                   unsigned *arrivals) {
+__global__ __launch_bounds__(kBeginThreads) void loop_begin_kernel(
+    KParams kp, Grid in, Grid other, int bc, StepCtl *ctl, double t, int nstep, double *partials,
+    unsigned *arrivals, double *host_rate) {
   using T = typename P::T;
   if (bc) {  // one thread per ghost cell of each array, as boundaries_kernel
     const int nghost = 4 * kp.isize + 4 * kp.ny;
@@ -653,22 +662,22 @@ __global__ __launch_bounds__(kBeginThreads) void loop_begin_kernel(KParams kp, G
       P::store(U, (long long)j * U.pitch + i, c);
     }
   }
-  // rows b, b + G, b + 2G, b + 3G loaded together, then converted
-  constexpr int kRows = 4;
   T m = T(0.0);
-  for (int j0 = 2 + blockIdx.x; j0 <= kp.ny + 1; j0 += kRows * gridDim.x)
-    for (int i = 2 + threadIdx.x; i <= kp.nx + 1; i += blockDim.x) {
-      typename P::Cell c[kRows];
+  const int lane = threadIdx.x & (kLanes - 1), waves = kBeginThreads / kLanes;
+  const int across = (kp.nx + kLanes - 1) / kLanes;
+  const int pieces = across * ((kp.ny + kBeginRows - 1) / kBeginRows);
+  for (int k = blockIdx.x * waves + (int)(threadIdx.x >> 6); k < pieces;
+       k += gridDim.x * waves) {
+    const int i = 2 + (k % across) * kLanes + lane, j0 = 2 + (k / across) * kBeginRows;
+    if (i > kp.nx + 1) continue;
+    typename P::Cell c[kBeginRows];
 #pragma unroll
-      for (int u = 0; u < kRows; u++) {
-        const int j = j0 + u * (int)gridDim.x;
-        if (j <= kp.ny + 1) c[u] = P::load(in, (long long)j * in.pitch + i);
-      }
+    for (int u = 0; u < kBeginRows; u++)
+      if (j0 + u <= kp.ny + 1) c[u] = P::load(in, (long long)(j0 + u) * in.pitch + i);
 #pragma unroll
-      for (int u = 0; u < kRows; u++) {
-        if (j0 + u * (int)gridDim.x <= kp.ny + 1) m = Ops<T>::mx(m, cell_rate<P>(kp, c[u]));
-      }
-    }
+    for (int u = 0; u < kBeginRows; u++)
+      if (j0 + u <= kp.ny + 1) m = Ops<T>::mx(m, cell_rate<P>(kp, c[u]));
+  }
   __shared__ double wm[kBeginThreads / kLanes];
   __shared__ bool last;
   const double md = wave_max(m);
@@ -701,10 +710,15 @@ __global__ __launch_bounds__(kBeginThreads) void loop_begin_kernel(KParams kp, G
   if (threadIdx.x < kRateSlots) {
     double mx = 0.0;
     for (int w = 0; w < (int)(blockDim.x / kLanes); w++) mx = wm[w] > mx ? wm[w] : mx;
+    if (host_rate) {
+      if (threadIdx.x == 0)
+        __hip_atomic_store(host_rate, mx, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+      return;
+    }
     ctl->rate[0][threadIdx.x * kSlotStride] = threadIdx.x == 0 ? dbits(mx) : 0ull;
     ctl->rate[1][threadIdx.x * kSlotStride] = 0ull;
   }
-  if (threadIdx.x == 0) {
+  if (threadIdx.x == 0 && !host_rate) {
     StepState s0;
     s0.t = t;
     s0.nstep = nstep;
@@ -2293,9 +2307,10 @@ hipError_t launch_fill_u32(unsigned *p, unsigned v, hipStream_t st) {
 }
 
 hipError_t launch_loop_begin(const KParams &kp, Grid in, Grid other, int bc, StepCtl *ctl,
-                             double t, int nstep, double *partials, hipStream_t st) {
-  E2D_DISPATCH_P(kp, loop_begin_kernel, dim3(kBeginBlocks), dim3(kBeginThreads), 0, st, kp, in,
-                 other, bc, ctl, t, nstep, partials, &ctl->arrivals);
+                             double t, int nstep, double *partials, hipStream_t st,
+                             double *host_rate) {
+  E2D_DISPATCH_P(kp, loop_begin_kernel, dim3((unsigned)begin_blocks(kp)), dim3(kBeginThreads), 0,
+                 st, kp, in, other, bc, ctl, t, nstep, partials, &ctl->arrivals, host_rate);
   return hipGetLastError();
 }
 

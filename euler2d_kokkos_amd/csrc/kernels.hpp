@@ -60,7 +60,7 @@ struct StepState {
   int nstep;  // steps executed before it
   int pad;
 };
-constexpr int kBeginBlocks = 512;  // blocks (and partials) of loop_begin_kernel
+constexpr int kBeginBlocks = 512;  // most blocks (and partials) of loop_begin_kernel
 constexpr int kRateSlots = 16;   // wavefront w folds into slot w % kRateSlots
 constexpr int kSlotStride = 16;  // one 128-byte line per slot
 struct StepCtl {
@@ -188,9 +188,11 @@ hipError_t launch_dt_reduce(const KParams &kp, Grid U, unsigned long long *invdt
                             hipStream_t st);
 // start of a run loop from (t, nstep): CFL rate of `in` into ring phase 0 of
 // *ctl, with `bc` also the ghost cells of `in` and `other`; partials holds
-// kBeginBlocks doubles
+// kBeginBlocks doubles.  host_rate: the rate goes to this pinned host word and the
+// rings stay as they are.
 hipError_t launch_loop_begin(const KParams &kp, Grid in, Grid other, int bc, StepCtl *ctl,
-                             double t, int nstep, double *partials, hipStream_t st);
+                             double t, int nstep, double *partials, hipStream_t st,
+                             double *host_rate = nullptr);
 // count of interior cells below the kinetic-energy threshold kp.kin_frac (added to *count)
 hipError_t launch_kinetic_count(const KParams &kp, Grid U, unsigned long long *count,
                                 hipStream_t st);
