@@ -487,8 +487,9 @@ int run_loop_impl(e2d_run *r, int max_steps, double *t, int *nStep, double *elap
 // buffers, two per host thread: while a thread copies one to (from) the caller's
 // array, the GPU fills (empties) the other.  Smaller chunks pay a launch and a
 // wait (about 10 us) too often, larger ones leave more of the first and last
-// chunk unoverlapped.
-constexpr size_t kStageChunk = 2u << 20;
+// chunk unoverlapped.  One thread takes 1 MiB (512x512, chunks of 0.5 / 1 / 2 MiB:
+// 0.47 / 0.32 / 0.39 ms), each of several 2 MiB.
+constexpr size_t kStageChunk = 1u << 20;
 // From 16 MiB on, four threads copy: one alone moves 13 GB/s into memory that the
 // caller has just allocated (page faults), PCIe about 50 GB/s.  A 1024x1536 state
 // (50 MB) takes 3.8 ms with one thread and 2.0 ms with four (57 ms as plane copies
@@ -497,7 +498,8 @@ constexpr size_t kStageChunk = 2u << 20;
 constexpr int kStageThreads = 4;
 constexpr size_t kStageThreadsFrom = 16u << 20;
 
-// `nbuf` pinned buffers of at least `bytes` bytes, with an event each
+// `nbuf` pinned buffers of at least `bytes` bytes, with an event each.  The buffers
+// only grow, in both respects (a batch's instances take turns with one set).
 hipError_t stage_reserve(Staging &s, size_t bytes, int nbuf) {
   for (int k = 0; k < nbuf; ++k)
     if (!s.ev[k]) {
@@ -505,6 +507,8 @@ hipError_t stage_reserve(Staging &s, size_t bytes, int nbuf) {
       if (e != hipSuccess) return e;
     }
   if (s.bytes >= bytes && s.nbuf >= nbuf) return hipSuccess;
+  bytes = std::max(bytes, s.bytes);
+  nbuf = std::max(nbuf, s.nbuf);
   if (s.host) (void)hipHostFree(s.host);
   s.host = nullptr;
   s.bytes = 0;
@@ -535,10 +539,12 @@ int stage_copy(const e2d_run *r, Staging &s, const Grid &g, double *host, int la
   const bool columns = layout == E2D_LAYOUT_RIGHT;
   const int units = columns ? box.ni : 4 * box.nj;
   const size_t unit = columns ? (size_t)box.nj * 32 : (size_t)box.ni * 8;
-  int per = (int)std::min<size_t>((size_t)units, std::max<size_t>(1, kStageChunk / unit));
+  const bool threads = unit * units >= kStageThreadsFrom;
+  const size_t chunk = threads ? 2 * kStageChunk : kStageChunk;
+  int per = (int)std::min<size_t>((size_t)units, std::max<size_t>(1, chunk / unit));
   if (columns && per < units && per > 16) per -= per % 16;  // whole tiles
   const int nchunks = (units + per - 1) / per;
-  const int nthreads = unit * units >= kStageThreadsFrom ? std::min(kStageThreads, nchunks) : 1;
+  const int nthreads = threads ? std::min(kStageThreads, nchunks) : 1;
   const hipError_t re = stage_reserve(s, unit * per, nchunks > 1 ? 2 * nthreads : 1);
   if (re != hipSuccess)
     return fail(E2D_ERR_ALLOC, std::string("staging buffers: ") + hipGetErrorString(re));
