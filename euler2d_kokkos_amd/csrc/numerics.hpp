@@ -82,8 +82,9 @@ struct SchemeT {
   T gamma0, gamma6, smallr, smallc, smallp, smallpp, slope_type, entho;
   T smallc2;    // smallc * smallc
   int riemann;  // 0 approx, 1 hll, 2 hllc (already resolved from honor_riemann)
-  // smallr and smallc >= 2^-60, smallr*smallp >= 2^-182, gamma0 <= 16, entho <= 2^20: the
-  // sound speeds take the short sqrt and the step's quotients the bounded forms
+  // smallr and smallc >= 2^-60, smallr*smallp >= 2^-182, gamma0 <= 16, entho <= 2^20, cell
+  // sizes of 2^-100 .. 2^100: the sound speeds take the short sqrt and the step's
+  // quotients the bounded forms
   int floor_sqrt;
 };
 using Scheme = SchemeT<double>;
@@ -164,6 +165,12 @@ __device__ __forceinline__ double quot_shared(double a, double d, double r, bool
   ok = ok && __builtin_amdgcn_class(q, kClassZeroOrNormal) &&
        __builtin_amdgcn_class(e, kClassZeroOrNormal);
   return __builtin_copysign(q, m);
+}
+
+// 2^lo <= x < 2^(hi + 1), for positive bounds: one comparison of the high word
+__device__ __forceinline__ bool exponent_within(double x, int lo, int hi) {
+  const unsigned h = (unsigned)(__double_as_longlong(x) >> 32);
+  return h - ((unsigned)(1023 + lo) << 20) < (unsigned)(hi - lo + 1) << 20;
 }
 
 // true in every lane when no active lane of the wavefront has !ok
@@ -332,7 +339,8 @@ __device__ __forceinline__ double cfl_rate_fp64(const Scheme &s, double u0, doub
   // bounded: smallp <= p / d <= 2^150, nothing to scale
   double x = FS ? quot_plain(s.gamma0 * q.v[IP], q.v[ID], r)
                 : quot_shared(s.gamma0 * q.v[IP], q.v[ID], r, rok);
-  if (!wave_all(ok && rok)) {  // uniform
+  const bool all = wave_all(ok && rok);
+  if (!all) {  // uniform
     prim_no_c<double, false>(s, u0, u1, u2, u3, q);
     x = (s.gamma0 * q.v[IP]) / q.v[ID];
   }
@@ -340,6 +348,19 @@ __device__ __forceinline__ double cfl_rate_fp64(const Scheme &s, double u0, doub
   const double vx = c + fabs(q.v[IU]);
   const double vy = c + fabs(q.v[IV]);
   if constexpr (POW2) return vx * rt.idx + vy * rt.idy;
+  if constexpr (FS) {
+    // The cell sizes' correctly rounded reciprocals are at hand: with them the
+    // residual step gives the IEEE quotient (Markstein 1990) wherever nothing
+    // leaves the normal range (speeds of 2^-62 .. 2^52 here, cell sizes of 2^-100 ..
+    // 2^100 by the host's floor_sqrt condition).  3 instructions instead of 11, one
+    // of them a reciprocal, per direction.
+    double rx = quot_plain(vx, rt.dx, rt.idx), ry = quot_plain(vy, rt.dy, rt.idy);
+    if (!all) {  // uniform
+      rx = vx / rt.dx;
+      ry = vy / rt.dy;
+    }
+    return rx + ry;
+  }
   double rx, ry;
   if (rt.pow2x)  // uniform
     rx = vx * rt.idx;
@@ -532,7 +553,7 @@ __device__ __forceinline__ T wave_speed(const SchemeT<T> &s, T pl, T rl, T pr, T
 // BND: the two quotients by rcr + rcl share a reciprocal, as do the two by
 // Sk - ustar; ok is cleared in a lane where one of them may differ from the
 // IEEE quotient.  Of the bounded ranges' consequences these are left to test:
-// rcr + rcl and Sk - ustar away from zero, and the residuals of ustar and
+// rcr + rcl (2^-150 .. 2^40) and Sk - ustar away from zero, and the residuals of ustar and
 // etotstar, whose numerators may be tiny (those of ptotstar and rstar are
 // zero or at least 2^-410; an overflow anywhere makes the last residual NaN
 // or infinite).  No numerator is ever -0: each ends in a sum with +0 or with a
@@ -564,7 +585,7 @@ __device__ __forceinline__ void hllc(const SchemeT<T> &s, const Q4T<T> &ql, cons
   T ustar, ptotstar;
   if constexpr (BND) {
     const T r = recip_newton(rc);
-    ok = ok && rc >= T(0x1p-150);
+    ok = ok && exponent_within(rc, -150, 40);
     ustar = quot_resid(un, rc, r, ok);
     ptotstar = quot_plain(pn, rc, r);
   } else {
