@@ -395,17 +395,18 @@ __device__ __forceinline__ float select_neg(bool neg, float z) { return neg ? -z
 template <bool MINMOD = false, class T>
 __device__ __forceinline__ T limited_slope(T st, T q, T qplus, T qminus) {
   using O = Ops<T>;
-  if constexpr (MINMOD && sizeof(T) == sizeof(double)) {
+  if constexpr (MINMOD) {
     // The sum of two one-sided differences of one sign is at least twice the
     // smaller, after rounding too, so |dcen| never limits them; and dcen >= 0
-    // where qplus >= qminus, except that qminus - qplus = 2^-1074 halves to -0:
-    // callers keep to values whose differences are zero or larger than that.
+    // where qplus >= qminus, except that the smallest denormal difference halves
+    // to -0: the FP64 callers keep to values whose differences are zero or larger
+    // (in FP32 the sign of that zero slope is the only change).
     const T dl = q - qminus, dr = qplus - q;
     const T z = (dl * dr <= T(0.0)) ? T(0.0) : O::mn(O::ab(dl), O::ab(dr));
     return select_neg(!(qplus >= qminus), z);
   }
-  const T dlft = MINMOD ? q - qminus : st * (q - qminus);
-  const T drgt = MINMOD ? qplus - q : st * (qplus - q);
+  const T dlft = st * (q - qminus);
+  const T drgt = st * (qplus - q);
   const T dcen = T(0.5) * (qplus - qminus);
   const T dsgn = (dcen >= T(0.0)) ? T(1.0) : T(-1.0);
   const T slop = O::mn(O::ab(dlft), O::ab(drgt));
@@ -769,8 +770,8 @@ constexpr int kRiemannFloorSqrt = 8;
 // cell sizes that are powers of two (its CFL rate); the host selects such a
 // kernel only then
 constexpr int kMinmodPow2 = 16;
-// + kSlopeMinmod: the march's slopes alone are built for slope_type == 1 (the
-// batch kernels, whose instances' cell sizes may be anything)
+// + kSlopeMinmod: the march's slopes alone are built for slope_type == 1 (any
+// cell sizes)
 constexpr int kSlopeMinmod = 32;
 // + kPruneRate: the march forms a cell's CFL rate only where it may exceed one
 // that the step has already found (bounded FP64 kinds, launches of more than two
