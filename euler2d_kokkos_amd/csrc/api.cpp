@@ -942,7 +942,7 @@ int e2d_kinetic_cells(e2d_run *r, int which, long long *count) {
   int rc = check_run(r);
   if (rc) return rc;
   if (!count || (which != E2D_U && which != E2D_U2)) return fail(E2D_ERR_ARG, "bad argument");
-  unsigned long long *dev = r->bits + 1;  // bits[0] is compute_dt's
+  unsigned long long *dev = r->bits;
   HIP_TRY(hipMemsetAsync(dev, 0, sizeof(unsigned long long), r->stream));
   HIP_TRY(e2d::launch_kinetic_count(r->kp, state(r, which), dev, r->stream));
   unsigned long long n = 0;
@@ -1166,7 +1166,10 @@ struct e2d_batch {
   e2d::StepCtl *ctls = nullptr;      // device, one per instance
   int phase = 0;                     // phase of the next launch in the control rings
   bool ready = false;                // e2d_batch_init has set every instance's loop state
-  int nwaves = 0;
+  e2d::BatchItem *items = nullptr;   // device: the work of one launch per step
+  size_t items_cap = 0;
+  int nitems = 0;
+  int nwaves = 0;                    // work items of a step of the persistent launch
   long long cells = 0;
   hipGraphExec_t graph = nullptr;
   int graph_steps = 0;
@@ -1283,6 +1286,7 @@ int batch_upload_table(e2d_batch *b) {
   int waves = 0;
   long long cells = 0;
   std::vector<int> inst_waves(b->runs.size());
+  std::vector<e2d::BatchItem> items;
   for (size_t i = 0; i < b->runs.size(); ++i) {
     e2d_run *r = b->runs[i];
     e2d::BatchInst &bi = h[i];
@@ -1290,19 +1294,35 @@ int batch_upload_table(e2d_batch *b) {
     bi.kp = r->kp;
     bi.U = r->U;
     bi.U2 = r->U2;
-    bi.wave_begin = waves;
     inst_waves[i] = e2d::batch_waves(r->kp, b->seg_rows, &bi.nstrips);
+    e2d::batch_items(r->kp, b->seg_rows, (int)i, items);
     waves += inst_waves[i];
     cells += (long long)r->p.nx * r->p.ny;
   }
   b->nwaves = waves;
   b->cells = cells;
+  e2d::batch_order(h.data(), items);
+  batch_drop_graph(b);
+  if (items.size() > b->items_cap) {
+    HIP_TRY(hipStreamSynchronize(b->stream));
+    if (b->items) (void)hipFree(b->items);
+    b->items = nullptr;
+    b->items_cap = 0;
+    b->nitems = 0;
+    void *ptr = nullptr;
+    if (hipMalloc(&ptr, items.size() * sizeof(e2d::BatchItem)) != hipSuccess)
+      return fail(E2D_ERR_ALLOC, "batch: device allocation failed");
+    b->items = static_cast<e2d::BatchItem *>(ptr);
+    b->items_cap = items.size();
+  }
+  HIP_TRY(hipMemcpyAsync(b->items, items.data(), items.size() * sizeof(e2d::BatchItem),
+                         hipMemcpyHostToDevice, b->stream));
+  b->nitems = (int)items.size();
   HIP_TRY(hipMemcpyAsync(b->insts, h.data(), h.size() * sizeof(e2d::BatchInst),
                          hipMemcpyHostToDevice, b->stream));
   int rc = batch_upload_queue(b, inst_waves);
   if (rc) return rc;
   HIP_TRY(hipStreamSynchronize(b->stream));
-  batch_drop_graph(b);
   return E2D_OK;
 }
 
@@ -1318,13 +1338,15 @@ int batch_tile(e2d_batch *b, int seg_rows) {
 // wavefront per SIMD (prefetch distance 1, short segments; tiles 14 / 20 / 48: 229 /
 // 218 / 222 us).
 int batch_auto_tile(const e2d_batch *b) {
+  const bool persistent = b->launch == E2D_BATCH_LAUNCH_PERSISTENT;
   auto waves = [&](int tile) {
     long long w = 0;
-    for (const e2d_run *r : b->runs) w += e2d::batch_waves(r->kp, tile, nullptr);
+    for (const e2d_run *r : b->runs)
+      w += persistent ? e2d::batch_waves(r->kp, tile, nullptr) : e2d::fused_map(r->kp, tile).nwaves;
     return (double)w;
   };
   const int simds = b->runs[0]->kp.simds;
-  if (b->launch == E2D_BATCH_LAUNCH_PERSISTENT) {
+  if (persistent) {
     if (b->precision != E2D_PRECISION_FP64) return 20;
     int tile = 16;
     while (tile < 64 && waves(tile) > 3.5 * simds) tile += 4;
@@ -1346,8 +1368,8 @@ int batch_launch(e2d_batch *b) {
   e2d::KParams k0 = b->runs[0]->kp;
   k0.s.floor_sqrt = b->floor_sqrt;
   for (const e2d_run *r : b->runs) k0.wide_addr |= r->kp.wide_addr;
-  HIP_TRY(e2d::launch_step_batch(k0, b->insts, (int)b->runs.size(), b->ctls, b->phase,
-                                 b->nwaves, b->seg_rows, b->stream, b->minmod != 0));
+  HIP_TRY(e2d::launch_step_batch(k0, b->insts, b->items, b->nitems, b->ctls, b->phase, b->stream,
+                                 b->minmod != 0));
   b->phase = b->phase == 2 ? 0 : b->phase + 1;
   return E2D_OK;
 }
@@ -1609,6 +1631,7 @@ int e2d_batch_destroy(e2d_batch *b) {
   for (e2d_run *r : b->runs) e2d_destroy(r);
   stage_release(b->staging);
   if (b->insts) (void)hipFree(b->insts);
+  if (b->items) (void)hipFree(b->items);
   if (b->ctls) (void)hipFree(b->ctls);
   if (b->queue_ints) (void)hipFree(b->queue_ints);
   if (b->counters) (void)hipFree(b->counters);
@@ -1644,7 +1667,7 @@ int e2d_batch_set_tile(e2d_batch *b, int seg_rows) {
   if (rc) return rc;
   if (seg_rows < 1 || seg_rows > 4096) return fail(E2D_ERR_ARG, "seg_rows must be in [1, 4096]");
   b->tile_chosen = true;
-  return batch_tile(b, seg_rows);
+  return guarded([&]() -> int { return batch_tile(b, seg_rows); });
 }
 
 int e2d_batch_run(e2d_batch *b, int max_steps, int use_graph, double *elapsed_ms,

@@ -1385,11 +1385,6 @@ __device__ __forceinline__ LoopPos loop_resolve(const KParams &kp, double t, int
   return L;
 }
 
-__device__ __forceinline__ LoopPos loop_pos(const KParams &kp, const StepCtl *ctl, int ph) {
-  const LoopWords w = loop_words(ctl, ph);
-  return loop_resolve(kp, w.t, w.nstep, w.slot);
-}
-
 // The step's one writer, the lanes of one wavefront: the state after the step
 // (main.cpp:143, t += dt and nStep++; unchanged once the loop has ended) and
 // the cleared rate entry of the launch after the next.  Nothing in this launch
@@ -1714,10 +1709,11 @@ void step_block_kernel(KParams kp, Grid in, Grid out, double dt_arg, StepCtl *ct
 // ------------------------------------------------------- batched step kernel
 //
 // One launch advances every active instance of a batch by one step, each with
-// its own dt.  Wavefront w works on the instance whose wave range contains w
-// (binary search over wave_begin), on that instance's strip / segment; its
-// in/out arrays follow the instance's own step parity.  Each instance has its
-// own loop control rings (StepCtl), published by its first wavefront.
+// its own dt.  A wavefront reads its item (instance, strip, segment) from a table:
+// one scalar load, where a search over the instances' first wavefronts was a chain of
+// six.  Its in/out arrays follow the instance's own step parity, and the loop's words
+// load beside the first rows.  Each instance has its own loop control rings
+// (StepCtl), published by the wavefront of its first segment.
 // Prefetch distance of the batch kernels: two rows ahead in FP64 (48 instances 88.1
 // -> 86.5 us a step, 192 instances 293 -> 288), one in the FP32 paths, which keep
 // their third wavefront per SIMD with it.
@@ -1725,60 +1721,50 @@ template <class P>
 constexpr int kBatchPrefetch = std::is_same<P, P64>::value ? 2 : 1;
 
 template <int RS, class P, bool O32>
-__device__ __forceinline__ void batch_step_wave(const BatchInst *__restrict__ insts, int ninst,
-                                                StepCtl *ctls, int ph, int nwaves,
-                                                int seg_rows) {
+__device__ __forceinline__ void batch_step_wave(const BatchInst *__restrict__ insts,
+                                                const BatchItem *__restrict__ items, int nitems,
+                                                StepCtl *ctls, int ph, bool prio) {
   using T = typename P::T;
   const int wave =
       __builtin_amdgcn_readfirstlane(blockIdx.x * (kBlock / kLanes) + (threadIdx.x >> 6));
-  T wmax = T(0.0);
-  unsigned long long *target = nullptr;
-  if (wave < nwaves) {
-    int lo = 0, hi = ninst - 1;
-    while (lo < hi) {  // last instance with wave_begin <= wave
-      const int mid = (lo + hi + 1) >> 1;
-      if (insts[mid].wave_begin <= wave)
-        lo = mid;
-      else
-        hi = mid - 1;
-    }
-    const int inst = __builtin_amdgcn_readfirstlane(lo);  // wave-uniform: scalar loads of the table
-    const BatchInst &bi = insts[inst];
-    StepCtl *ctl = ctls + inst;
-    // by-value copies: the march then reads its parameters from scalar
-    // registers instead of reloading them around every store
-    const KParams kp = bi.kp;
-    const LoopPos L = loop_pos(kp, ctl, ph);
-    const int w = wave - bi.wave_begin;
-    if (w == 0) loop_publish(ctl, ph, L, threadIdx.x & (kLanes - 1));
-    if (L.active) {
-      const bool even = (L.nstep & 1) == 0;
-      // U and U2 share their geometry (one allocation shape per instance)
-      const Grid gin = even ? bi.U : bi.U2;
-      Grid gout = gin;
-      gout.p = even ? bi.U2.p : bi.U.p;
-      const int strip = w % bi.nstrips, seg = w / bi.nstrips;
-      auto start = [&](double &dt) -> bool {
-        dt = L.dt;
-        return true;
-      };
-      if (interior_cols(kp, strip))
-        wmax = march<RS, P, true, O32, false, kBatchPrefetch<P>>(kp, gin, gout, start, seg_rows, bi.nstrips,
-                                              strip, seg, false, 0.0f);
-      else
-        wmax = march<RS, P, true, O32, true, kBatchPrefetch<P>>(kp, gin, gout, start, seg_rows, bi.nstrips,
-                                             strip, seg, false, 0.0f);
-      target = rate_slot(ctl, ph);
-    }
-  }
-  reduce_rate_wave(wmax, target);
+  if (wave >= nitems) return;
+  const BatchItem it = items[wave];
+  const BatchInst &bi = insts[it.inst];
+  StepCtl *ctl = ctls + it.inst;
+  const LoopWords words = loop_words(ctl, ph);
+  // by-value copies: the march then reads its parameters from scalar
+  // registers instead of reloading them around every store
+  const KParams kp = bi.kp;
+  const bool even = (words.nstep & 1) == 0;
+  // U and U2 share their geometry (one allocation shape per instance)
+  const Grid gin = even ? bi.U : bi.U2;
+  Grid gout = gin;
+  gout.p = even ? bi.U2.p : bi.U.p;
+  bool go = true;
+  auto start = [&](double &dt) -> bool {
+    const LoopPos L = loop_resolve(kp, words.t, words.nstep, words.slot);
+    if (it.strip == 0 && it.seg == 0) loop_publish(ctl, ph, L, threadIdx.x & (kLanes - 1));
+    go = L.active;  // false once the instance's loop has finished
+    dt = L.dt;
+    return go;
+  };
+  T wmax;
+  if (interior_cols(kp, it.strip))
+    wmax = march<RS, P, true, O32, false, kBatchPrefetch<P>>(kp, gin, gout, start, it.rows,
+                                                             bi.nstrips, it.strip, it.seg, prio,
+                                                             0.0f);
+  else
+    wmax = march<RS, P, true, O32, true, kBatchPrefetch<P>>(kp, gin, gout, start, it.rows,
+                                                            bi.nstrips, it.strip, it.seg, prio,
+                                                            0.0f);
+  if (go) reduce_rate_wave(wmax, rate_slot(ctl, ph));
 }
 
 template <int RS, class P, bool O32>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(2)))
-void step_batch_kernel(const BatchInst *__restrict__ insts, int ninst, StepCtl *ctls, int ph,
-                       int nwaves, int seg_rows) {
-  batch_step_wave<RS, P, O32>(insts, ninst, ctls, ph, nwaves, seg_rows);
+void step_batch_kernel(const BatchInst *__restrict__ insts, const BatchItem *__restrict__ items,
+                       int nitems, StepCtl *ctls, int ph, int prio) {
+  batch_step_wave<RS, P, O32>(insts, items, nitems, ctls, ph, prio != 0);
 }
 
 // The split-precision step held to three wavefronts per SIMD (168 VGPRs, a few
@@ -1787,9 +1773,10 @@ void step_batch_kernel(const BatchInst *__restrict__ insts, int ninst, StepCtl *
 // 512-instance sweep.
 template <int RS, class P, bool O32>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(3)))
-void step_batch_kernel_w3(const BatchInst *__restrict__ insts, int ninst, StepCtl *ctls, int ph,
-                          int nwaves, int seg_rows) {
-  batch_step_wave<RS, P, O32>(insts, ninst, ctls, ph, nwaves, seg_rows);
+void step_batch_kernel_w3(const BatchInst *__restrict__ insts,
+                          const BatchItem *__restrict__ items, int nitems, StepCtl *ctls, int ph,
+                          int prio) {
+  batch_step_wave<RS, P, O32>(insts, items, nitems, ctls, ph, prio != 0);
 }
 
 // ----------------------------------------------- persistent batched step kernel
@@ -2082,6 +2069,11 @@ bool off32_ok(const KParams &kp, const Grid &g) {
 
 dim3 grid2d(int nx, int ny, dim3 blk) {
   return dim3((unsigned)((nx + blk.x - 1) / blk.x), (unsigned)((ny + blk.y - 1) / blk.y));
+}
+
+// every wavefront resident at once, two per SIMD (FusedMap::prio)
+int two_resident(int nwaves, int simds) {
+  return simds > 0 && nwaves > simds && nwaves <= 2 * simds ? 1 : 0;
 }
 
 template <int RS, class P>
@@ -2490,8 +2482,37 @@ FusedMap fused_map(const KParams &kp, int seg_rows) {
   const int nsegs_e = (kp.ny + f.tile_e - 1) / f.tile_e;
   f.n_int = (f.nstrips - f.nedge) * nsegs_i;
   f.nwaves = f.n_int + f.nedge * nsegs_e;
-  f.prio = kp.simds > 0 && f.nwaves > kp.simds && f.nwaves <= 2 * kp.simds ? 1 : 0;
+  f.prio = two_resident(f.nwaves, kp.simds);
   return f;
+}
+
+// The segments of a strip are of nearly equal length (64 rows at a 27-row tile: 22, 22,
+// 20 and not 27, 27, 10), and those of edge strips shorter, as in the single grid's step.
+// With the longest launched first and, where all wavefronts are resident, the priority
+// that falls with progress, a SIMD's two wavefronts end closer together.  us per step,
+// uniform segments in instance order -> these: 8 instances FP64 27.5 -> 25.5, split
+// 18.8 -> 17.0; 24: 45.2 -> 41.3, 30.2 -> 27.4; 48: 86 -> 79, 55.7 -> 49; 192: 308 -> 291,
+// 240 -> 237.
+void batch_items(const KParams &kp, int seg_rows, int inst, std::vector<BatchItem> &items) {
+  const FusedMap f = fused_map(kp, seg_rows);
+  auto add = [&](int first, int count, int stride, int tile) {
+    const int n = (kp.ny + tile - 1) / tile;
+    const int rows = (kp.ny + n - 1) / n;
+    for (int seg = 0; seg * rows < kp.ny; ++seg)
+      for (int k = 0; k < count; ++k) items.push_back(BatchItem{inst, first + k * stride, seg, rows});
+  };
+  add(1, f.nstrips - f.nedge, 1, f.tile);
+  add(0, f.nedge, f.nstrips - 1, f.tile_e);
+}
+
+void batch_order(const BatchInst *insts, std::vector<BatchItem> &items) {
+  auto cost = [&](const BatchItem &it) {
+    const bool edge = it.strip == 0 || it.strip == insts[it.inst].nstrips - 1;
+    return (it.rows + 4) * (edge ? 11 : 10);
+  };
+  std::stable_sort(items.begin(), items.end(), [&](const BatchItem &a, const BatchItem &b) {
+    return cost(a) > cost(b);
+  });
 }
 
 int batch_waves(const KParams &kp, int seg_rows, int *nstrips) {
@@ -2564,19 +2585,20 @@ hipError_t launch_step_batch_persistent(const KParams &kp0, const BatchInst *ins
 #undef E2D_PBATCH_ARGS
 }
 
-hipError_t launch_step_batch(const KParams &kp0, const BatchInst *insts_dev, int ninst,
-                             StepCtl *ctls_dev, int ph, int nwaves, int seg_rows, hipStream_t st,
-                             bool minmod) {
-  if (ph < 0 || ph > 2) return hipErrorInvalidValue;
-  const int blocks = (nwaves + kBlock / kLanes - 1) / (kBlock / kLanes);
+hipError_t launch_step_batch(const KParams &kp0, const BatchInst *insts_dev,
+                             const BatchItem *items_dev, int nitems, StepCtl *ctls_dev, int ph,
+                             hipStream_t st, bool minmod) {
+  if (ph < 0 || ph > 2 || nitems <= 0) return hipErrorInvalidValue;
+  const int blocks = (nitems + kBlock / kLanes - 1) / (kBlock / kLanes);
+  const int prio = two_resident(nitems, kp0.simds);
 #define E2D_BATCH_LAUNCH(K, RS, P)                                                            \
   do {                                                                                        \
     if (kp0.wide_addr)                                                                        \
       hipLaunchKernelGGL((K<RS, P, false>), dim3(blocks), dim3(kBlock), 0, st, insts_dev,     \
-                         ninst, ctls_dev, ph, nwaves, seg_rows);                               \
+                         items_dev, nitems, ctls_dev, ph, prio);                               \
     else                                                                                      \
       hipLaunchKernelGGL((K<RS, P, true>), dim3(blocks), dim3(kBlock), 0, st, insts_dev,      \
-                         ninst, ctls_dev, ph, nwaves, seg_rows);                               \
+                         items_dev, nitems, ctls_dev, ph, prio);                               \
   } while (0)
   if (kp0.prec == E2D_PRECISION_FP32_SPLIT) {
     if (minmod && kp0.s.riemann == 2)

@@ -4,6 +4,7 @@
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
+#include <vector>
 
 #include "euler2d_hip.h"
 #include "numerics.hpp"
@@ -80,9 +81,14 @@ struct StepCtl {
 struct BatchInst {
   KParams kp;
   Grid U, U2;
-  int wave_begin;  // first global wavefront index of this instance
   int nstrips;
-  int pad[2];
+  int pad[3];
+};
+
+// One wavefront's work in the batched step of one launch: segment `seg` of `rows`
+// rows of strip `strip` of instance `inst`.
+struct alignas(16) BatchItem {
+  int inst, strip, seg, rows;
 };
 
 // Work queues of the persistent batched step.  Every instance is assigned to
@@ -216,15 +222,20 @@ hipError_t launch_step_fused(const KParams &kp, Grid in, Grid out, double dt, St
                              int ph, int seg_rows, hipStream_t st);
 hipError_t launch_sums(const KParams &kp, Grid U, double *partials, double *out4, hipStream_t st);
 int sums_partials_needed(const KParams &kp);
-// wavefronts the fused step launches for one grid (and its strip count)
+// work items of one instance and step in the persistent launch (and its strip count)
 int batch_waves(const KParams &kp, int seg_rows, int *nstrips);
+// appends instance `inst`'s items of one step in the one-launch-per-step mode, at most
+// seg_rows rows each
+void batch_items(const KParams &kp, int seg_rows, int inst, std::vector<BatchItem> &items);
+// the order in which they are launched: those that take longest first
+void batch_order(const BatchInst *insts, std::vector<BatchItem> &items);
 // one step of every active instance; kp0 gives the precision and solver of all
 // (kp0.s.floor_sqrt must hold for every instance; kp0.wide_addr must be set
 // when any instance has a plane above 4 GiB; minmod: every instance has
 // slope_type 1)
-hipError_t launch_step_batch(const KParams &kp0, const BatchInst *insts_dev, int ninst,
-                             StepCtl *ctls_dev, int ph, int nwaves, int seg_rows, hipStream_t st,
-                             bool minmod = false);
+hipError_t launch_step_batch(const KParams &kp0, const BatchInst *insts_dev,
+                             const BatchItem *items_dev, int nitems, StepCtl *ctls_dev, int ph,
+                             hipStream_t st, bool minmod = false);
 // All `steps` steps of every instance in one persistent launch: as many blocks
 // of 256 threads as the kernel fits on `ncu` CUs at once.  counters and done
 // (one word every kCounterStride per instance) must be zero; steps times the
