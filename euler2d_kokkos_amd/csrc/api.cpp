@@ -130,20 +130,26 @@ int alloc_dev(e2d_run *r, void **ptr, size_t bytes) {
   return E2D_OK;
 }
 
-// Rows start on 128-byte and planes on 512-byte boundaries.
-int alloc_grid(e2d_run *r, Grid &g, int precision) {
+// The shape of a state array: rows start on 128-byte and planes on 512-byte boundaries.
+Grid grid_shape(const e2d_params &p, int precision) {
   const int sb = e2d::grid_scalar_bytes(precision);
   const int row_align = 128 / sb, plane_align = 512 / sb;
-  const int pitch = (r->p.isize + row_align - 1) / row_align * row_align;
-  long long plane = (long long)pitch * r->p.jsize;
-  plane = (plane + plane_align - 1) / plane_align * plane_align;
-  void *ptr = nullptr;
-  int rc = alloc_dev(r, &ptr, (size_t)plane * e2d::grid_planes(precision) * sb);
-  if (rc) return rc;
-  g.p = ptr;
-  g.pitch = pitch;
-  g.plane = plane;
-  return E2D_OK;
+  Grid g{};
+  g.pitch = (p.isize + row_align - 1) / row_align * row_align;
+  g.plane = (long long)g.pitch * p.jsize;
+  g.plane = (g.plane + plane_align - 1) / plane_align * plane_align;
+  return g;
+}
+
+size_t grid_bytes(const Grid &g, int precision) {
+  return (size_t)g.plane * e2d::grid_planes(precision) * e2d::grid_scalar_bytes(precision);
+}
+
+int alloc_grid(e2d_run *r, Grid &g, int precision) {
+  Grid n = grid_shape(r->p, precision);
+  int rc = alloc_dev(r, &n.p, grid_bytes(n, precision));
+  if (!rc) g = n;
+  return rc;
 }
 
 Grid &state(e2d_run *r, int which) { return which == E2D_U ? r->U : r->U2; }
@@ -613,6 +619,113 @@ int guarded(F &&f) {
   }
 }
 
+// What e2d_create and e2d_batch_create refuse before any GPU work.
+int check_create(const e2d_params &p, int precision) {
+  const int rc = e2d_params_validate(&p);
+  if (rc) return rc;
+  if (precision != E2D_PRECISION_FP64 && precision != E2D_PRECISION_FP32_SPLIT &&
+      precision != E2D_PRECISION_FP32)
+    return fail(E2D_ERR_ARG, "precision must be one of E2D_PRECISION_FP64 / _FP32_SPLIT / _FP32");
+  return E2D_OK;
+}
+
+int check_device() {
+  int ndev = 0;
+  const hipError_t e = hipGetDeviceCount(&ndev);
+  return e != hipSuccess || ndev == 0 ? fail(E2D_ERR_HIP, "no HIP device visible") : E2D_OK;
+}
+
+// The batch's state arrays lie one after the other in one allocation, kArenaGap bytes
+// apart.  Allocated one by one they all start on 2 MiB boundaries, and the wavefronts
+// of a step, which march up their segments together, meet in the same memory
+// channels: 48 instances, split precision, 61 us a step, 49 in one allocation (61 again
+// with 2 MiB alignment there).  The gap keeps arrays whose size is a multiple of 2 MiB
+// apart as well.
+constexpr size_t kArenaGap = 9 * 512;
+
+size_t arena_stride(const Grid &g, int precision) { return grid_bytes(g, precision) + kArenaGap; }
+
+// A handle whose U and U2 are allocated (arrays == nullptr), or lie at `arrays` and
+// arena_stride() further on.
+int create_run(const e2d_params *p, int precision, char *arrays, e2d_run **out) {
+  *out = nullptr;
+  int rc = check_create(*p, precision);
+  if (rc) return rc;
+  return guarded([&]() -> int {
+    rc = check_device();
+    if (rc) return rc;
+    auto *r = new e2d_run();
+    // every failure past this point releases what the handle holds
+    const int rc1 = [&]() -> int {
+    r->p = *p;
+    r->kp = e2d::make_kparams(*p, precision);
+    r->precision = precision;
+    // implementationVersion selects the schedule, as in godunov_unsplit_impl
+    // (HydroRun.h:312-357); version 0 runs fused, with the same bits
+    if (precision == E2D_PRECISION_FP64 && p->implementationVersion == 1)
+      r->schedule = E2D_SCHEDULE_DIRECTIONAL;
+    else if (precision == E2D_PRECISION_FP64 && p->implementationVersion == 2)
+      r->schedule = E2D_SCHEDULE_ATOMIC;
+    HIP_TRY(hipGetDevice(&r->device));
+    int ncu = 0;
+    HIP_TRY(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, r->device));
+    r->kp.simds = 4 * ncu;
+    r->seg_rows = e2d::auto_tile(r->kp);
+    HIP_TRY(hipStreamCreateWithFlags(&r->stream, hipStreamNonBlocking));
+    void *ptr = nullptr;
+    int rc2 = E2D_OK;
+    if (arrays) {
+      r->U = r->U2 = grid_shape(r->p, precision);
+      r->U.p = arrays;
+      r->U2.p = arrays + arena_stride(r->U, precision);
+    } else {
+      rc2 = alloc_grid(r, r->U, precision);
+      if (!rc2) rc2 = alloc_grid(r, r->U2, precision);
+    }
+    if (!rc2) rc2 = alloc_dev(r, &ptr, sizeof(e2d::StepCtl));
+    if (!rc2) r->ctl = static_cast<e2d::StepCtl *>(ptr);
+    if (!rc2) rc2 = alloc_dev(r, &ptr, 64);
+    if (!rc2) r->bits = static_cast<unsigned long long *>(ptr);
+    if (!rc2) rc2 = alloc_dev(r, &ptr, 64);
+    if (!rc2) r->count = static_cast<unsigned int *>(ptr);
+    if (!rc2) rc2 = alloc_dev(r, &ptr, (size_t)e2d::sums_partials_needed(r->kp) * sizeof(double));
+    if (!rc2) r->partials = static_cast<double *>(ptr);
+    if (!rc2) rc2 = alloc_dev(r, &ptr, 4 * sizeof(double));
+    if (!rc2) r->sums4 = static_cast<double *>(ptr);
+    if (rc2) return rc2;
+    HIP_TRY(hipEventCreate(&r->ev0));
+    HIP_TRY(hipEventCreate(&r->ev1));
+    const size_t host_bytes = 3 * sizeof(e2d::StepState) + sizeof(double);
+    HIP_TRY(hipHostMalloc(reinterpret_cast<void **>(&r->host_s), host_bytes,
+                          hipHostMallocDefault));
+    std::memset(r->host_s, 0, host_bytes);
+    r->host_rate = reinterpret_cast<double *>(r->host_s + 3);
+    // 32-bit row offsets in the step kernels need planes of at most 4 GiB;
+    // E2D_WIDE_ADDRESSING=1 selects the 64-bit form for any size
+    const char *wide = std::getenv("E2D_WIDE_ADDRESSING");
+    r->kp.wide_addr = (wide && *wide && std::strcmp(wide, "0") != 0) ||
+                      (unsigned long long)r->U.plane * e2d::grid_scalar_bytes(precision) >
+                          (1ull << 32);
+    // defined contents everywhere (ghosts included) before the first init
+    const size_t bytes = grid_bytes(r->U, precision);
+    HIP_TRY(hipMemsetAsync(r->U.p, 0, bytes, r->stream));
+    HIP_TRY(hipMemsetAsync(r->U2.p, 0, bytes, r->stream));
+    HIP_TRY(hipMemsetAsync(r->ctl, 0, sizeof(e2d::StepCtl), r->stream));
+    HIP_TRY(hipMemcpyAsync(&r->ctl->host_s, &r->host_s, sizeof(r->host_s), hipMemcpyHostToDevice,
+                           r->stream));
+    HIP_TRY(hipStreamSynchronize(r->stream));
+    return E2D_OK;
+    }();
+    if (rc1) {
+      const std::string msg = g_last_error;
+      e2d_destroy(r);
+      return fail(rc1, msg);
+    }
+    *out = r;
+    return E2D_OK;
+  });
+}
+
 }  // namespace
 
 extern "C" {
@@ -741,80 +854,7 @@ int e2d_params_validate(const e2d_params *p) {
 // --------------------------------------------------------------- HydroRun
 int e2d_create(const e2d_params *p, int precision, e2d_run **out) {
   if (!p || !out) return fail(E2D_ERR_ARG, "null argument");
-  *out = nullptr;
-  int rc = e2d_params_validate(p);
-  if (rc) return rc;
-  if (precision != E2D_PRECISION_FP64 && precision != E2D_PRECISION_FP32_SPLIT &&
-      precision != E2D_PRECISION_FP32)
-    return fail(E2D_ERR_ARG, "precision must be one of E2D_PRECISION_FP64 / _FP32_SPLIT / _FP32");
-  return guarded([&]() -> int {
-    int ndev = 0;
-    hipError_t e = hipGetDeviceCount(&ndev);
-    if (e != hipSuccess || ndev == 0) return fail(E2D_ERR_HIP, "no HIP device visible");
-    auto *r = new e2d_run();
-    // every failure past this point releases what the handle holds
-    const int rc1 = [&]() -> int {
-    r->p = *p;
-    r->kp = e2d::make_kparams(*p, precision);
-    r->precision = precision;
-    // implementationVersion selects the schedule, as in godunov_unsplit_impl
-    // (HydroRun.h:312-357); version 0 runs fused, with the same bits
-    if (precision == E2D_PRECISION_FP64 && p->implementationVersion == 1)
-      r->schedule = E2D_SCHEDULE_DIRECTIONAL;
-    else if (precision == E2D_PRECISION_FP64 && p->implementationVersion == 2)
-      r->schedule = E2D_SCHEDULE_ATOMIC;
-    HIP_TRY(hipGetDevice(&r->device));
-    int ncu = 0;
-    HIP_TRY(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, r->device));
-    r->kp.simds = 4 * ncu;
-    r->seg_rows = e2d::auto_tile(r->kp);
-    HIP_TRY(hipStreamCreateWithFlags(&r->stream, hipStreamNonBlocking));
-    void *ptr = nullptr;
-    int rc2 = alloc_grid(r, r->U, precision);
-    if (!rc2) rc2 = alloc_grid(r, r->U2, precision);
-    if (!rc2) rc2 = alloc_dev(r, &ptr, sizeof(e2d::StepCtl));
-    if (!rc2) r->ctl = static_cast<e2d::StepCtl *>(ptr);
-    if (!rc2) rc2 = alloc_dev(r, &ptr, 64);
-    if (!rc2) r->bits = static_cast<unsigned long long *>(ptr);
-    if (!rc2) rc2 = alloc_dev(r, &ptr, 64);
-    if (!rc2) r->count = static_cast<unsigned int *>(ptr);
-    if (!rc2) rc2 = alloc_dev(r, &ptr, (size_t)e2d::sums_partials_needed(r->kp) * sizeof(double));
-    if (!rc2) r->partials = static_cast<double *>(ptr);
-    if (!rc2) rc2 = alloc_dev(r, &ptr, 4 * sizeof(double));
-    if (!rc2) r->sums4 = static_cast<double *>(ptr);
-    if (rc2) return rc2;
-    HIP_TRY(hipEventCreate(&r->ev0));
-    HIP_TRY(hipEventCreate(&r->ev1));
-    const size_t host_bytes = 3 * sizeof(e2d::StepState) + sizeof(double);
-    HIP_TRY(hipHostMalloc(reinterpret_cast<void **>(&r->host_s), host_bytes,
-                          hipHostMallocDefault));
-    std::memset(r->host_s, 0, host_bytes);
-    r->host_rate = reinterpret_cast<double *>(r->host_s + 3);
-    // 32-bit row offsets in the step kernels need planes of at most 4 GiB;
-    // E2D_WIDE_ADDRESSING=1 selects the 64-bit form for any size
-    const char *wide = std::getenv("E2D_WIDE_ADDRESSING");
-    r->kp.wide_addr = (wide && *wide && std::strcmp(wide, "0") != 0) ||
-                      (unsigned long long)r->U.plane * e2d::grid_scalar_bytes(precision) >
-                          (1ull << 32);
-    // defined contents everywhere (ghosts included) before the first init
-    const size_t bytes =
-      (size_t)r->U.plane * e2d::grid_planes(precision) * e2d::grid_scalar_bytes(precision);
-    HIP_TRY(hipMemsetAsync(r->U.p, 0, bytes, r->stream));
-    HIP_TRY(hipMemsetAsync(r->U2.p, 0, bytes, r->stream));
-    HIP_TRY(hipMemsetAsync(r->ctl, 0, sizeof(e2d::StepCtl), r->stream));
-    HIP_TRY(hipMemcpyAsync(&r->ctl->host_s, &r->host_s, sizeof(r->host_s), hipMemcpyHostToDevice,
-                           r->stream));
-    HIP_TRY(hipStreamSynchronize(r->stream));
-    return E2D_OK;
-    }();
-    if (rc1) {
-      const std::string msg = g_last_error;
-      e2d_destroy(r);
-      return fail(rc1, msg);
-    }
-    *out = r;
-    return E2D_OK;
-  });
+  return create_run(p, precision, nullptr, out);
 }
 
 int e2d_destroy(e2d_run *run) {
@@ -1162,6 +1202,7 @@ struct e2d_batch {
   int seg_rows = 14;
   int device = 0;
   hipStream_t stream = nullptr;
+  char *arena = nullptr;             // device: the instances' state arrays
   e2d::BatchInst *insts = nullptr;   // device
   e2d::StepCtl *ctls = nullptr;      // device, one per instance
   int phase = 0;                     // phase of the next launch in the control rings
@@ -1522,9 +1563,31 @@ int e2d_batch_create(const e2d_params *params, int count, int precision, e2d_bat
   return guarded([&]() -> int {
     auto *b = new e2d_batch();
     b->precision = precision;
+    size_t total = 0;
+    for (int i = 0; i < count; ++i) {
+      int rc = check_create(params[i], precision);
+      if (rc) {
+        const std::string msg = "instance " + std::to_string(i) + ": " + g_last_error;
+        e2d_batch_destroy(b);
+        return fail(rc, msg);
+      }
+      total += 2 * arena_stride(grid_shape(params[i], precision), precision);
+    }
+    if (int rc = check_device()) {
+      e2d_batch_destroy(b);
+      return rc;
+    }
+    void *arena = nullptr;
+    if (hipMalloc(&arena, total) != hipSuccess) {  // one by one, then
+      arena = nullptr;
+      (void)hipGetLastError();
+    }
+    b->arena = static_cast<char *>(arena);
+    size_t at = 0;
     for (int i = 0; i < count; ++i) {
       e2d_run *r = nullptr;
-      int rc = e2d_create(params + i, precision, &r);
+      int rc = create_run(params + i, precision, b->arena ? b->arena + at : nullptr, &r);
+      at += 2 * arena_stride(grid_shape(params[i], precision), precision);
       if (rc) {
         const std::string msg = "instance " + std::to_string(i) + ": " + g_last_error;
         e2d_batch_destroy(b);
@@ -1630,6 +1693,7 @@ int e2d_batch_destroy(e2d_batch *b) {
   batch_drop_graph(b);
   for (e2d_run *r : b->runs) e2d_destroy(r);
   stage_release(b->staging);
+  if (b->arena) (void)hipFree(b->arena);
   if (b->insts) (void)hipFree(b->insts);
   if (b->items) (void)hipFree(b->items);
   if (b->ctls) (void)hipFree(b->ctls);
