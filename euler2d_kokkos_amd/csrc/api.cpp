@@ -1393,6 +1393,7 @@ int batch_auto_tile(const e2d_batch *b) {
     while (tile < 64 && waves(tile) > 3.5 * simds) tile += 4;
     return tile;
   }
+  if (e2d::many_rounds_split(b->runs[0]->kp, waves(e2d::kSplitTile))) return e2d::kSplitTile;
   int best = 14;
   double least = 1e300;
   for (int tile = 4; tile <= 64; ++tile) {

@@ -173,6 +173,13 @@ BlockMap block_map(const KParams &kp, int seg_rows);
 // 51.0 / 52.8 / 59.2 / 43.6 / 49.5 / 55.8 us; 3001x1777, tiles 14 / 24 / 48: 118 / 104 / 100
 // units, 160 / 154 / 144 us.
 double march_cost(double waves, int tile, int simds);
+// Split precision over more than eight rounds of wavefronts (counted at kSplitTile rows)
+// is bound by memory: short segments keep more of the halo rows in the caches than the
+// cost's longer ones.  8192x8192, 14 / 60 rows: 1022 / 1078 us a step; 16384x8192 2011 /
+// 2062; 4096x4096 266 / 271; 192 grids of 64 .. 512 219 / 235.  At six rounds (3001x1777)
+// the cost's tile wins: 85.8 against 90.7.
+constexpr int kSplitTile = 14;
+bool many_rounds_split(const KParams &kp, double waves);
 // The tile a run starts with: the smallest whose blocks fit one per CU (a
 // smaller one shortens each wavefront's chain as long as no second round of
 // blocks is needed: 256x256, tiles 6 / 8 / 12: 8.1 / 8.5 / 10.1 us); for larger
