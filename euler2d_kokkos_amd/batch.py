@@ -1,5 +1,5 @@
 """Batched driver: many independent instances advanced together, in one
-persistent launch per run (the default) or one launch per step.
+persistent launch per run (the default for many) or one launch per step.
 
 HydroBatch wraps the e2d_batch_* C ABI.  sweep_params() builds the seeded
 512-instance sweep: sizes nx, ny drawn independently from
@@ -95,7 +95,8 @@ class HydroBatch:
 
     def set_launch(self, mode: int, spin_limit: int = 0) -> None:
         """E2D_BATCH_LAUNCH_PERSISTENT (all the steps of a run in one launch;
-        the default when the instances fill the XCD queues evenly) or
+        the default when the instances fill the XCD queues evenly, at least 12
+        in each) or
         E2D_BATCH_LAUNCH_STEPS (one launch per step, replayed from hipGraphs;
         the default otherwise); spin_limit bounds each dependency wait of the
         persistent launch."""
