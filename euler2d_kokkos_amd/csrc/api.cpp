@@ -1263,9 +1263,9 @@ constexpr unsigned kDefaultSpinLimit = 1u << 20;
 // A new batch defaults to the persistent launch where its instances fill the XCD
 // queues evenly (fullest queue's cells over the mean) and each queue holds enough
 // of them that a wavefront hardly ever waits for its instance's previous step.
-// us per step, one launch per step / persistent, best tiles: 48 instances (6 a
-// queue, 2.7 Mcell) FP64 94 / 103, split 56 / 78; 96 (12 a queue) 185 / 177, 122 / 116;
-// 192: 333 / 316, 226 / 218.
+// us per step, one launch per step / persistent, default tiles: 48 instances (6 a
+// queue) FP64 84 / 113, split 50 / 92; 72: 123 / 133, 94 / 92; 96 (12 a queue) 170 / 170,
+// 121 / 112; 192: 312 / 300, 220 / 213; 512: 817 / 788, 566 / 566.
 constexpr double kPersistentImbalance = 1.10;
 constexpr int kPersistentPerQueue = 12;
 
