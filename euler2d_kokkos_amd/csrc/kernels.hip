@@ -973,13 +973,15 @@ enum : int {
 
 // The CFL rate of a step is the maximum over its cells, and the exact FP64 rate
 // of a cell costs a reciprocal, a square root and 90 instructions in all.  This
-// test costs 27, most of them FP32: a bound from above on the cell's rate, below a
+// test costs 28, most of them FP32: a bound from above on the cell's rate, below a
 // rate already found.  The conversion's rounding errors are within 2^-21
 // (|E| / d + v^2) in the specific internal energy, which the 2^-19 term covers,
 // and within 2^-20 relative in everything else, which the factor in the inverse
-// cell sizes covers.  Densities whose FP32 reciprocal could underflow, and values
-// outside FP32's range (infinity or NaN), are never below.  Cells that pass cannot
-// exceed a rate that takes part in the maximum, so the maximum keeps its bits.
+// cell sizes covers; what underflows in FP32 is covered by bound_floor.  Densities
+// whose reciprocal could underflow, speeds above 2^50 (whose square could leave
+// FP32's range and take the sound speed out of the bound) and energies past FP32's
+// range are never below.  Cells that pass cannot exceed a rate that takes part in
+// the maximum, so the maximum keeps its bits.
 __device__ __forceinline__ bool rate_below(const KParams &kp, const double u[4], float found) {
   const float d = fmaxf((float)u[0], kp.sf.smallr);
   const float r = __builtin_amdgcn_rcpf(d);
@@ -989,7 +991,7 @@ __device__ __forceinline__ bool rate_below(const KParams &kp, const double u[4],
   const float em = __builtin_fmaf(fabsf(e1) + k, 0x1p-19f, e);
   const float c = __builtin_amdgcn_sqrtf(fmaxf(kp.bound_c2 * em, kp.bound_floor));
   const float bound = __builtin_fmaf(c + fabsf(vx), kp.bound_idx, (c + fabsf(vy)) * kp.bound_idy);
-  return bound < found && d <= 0x1p100f;
+  return bound < found && d <= 0x1p100f && k <= 0x1p100f;
 }
 
 // a finite float below the rate
@@ -2272,7 +2274,11 @@ KParams make_kparams(const e2d_params &p, int precision) {
   // rate_below's constants: the last factor of its margin is in the cell sizes
   // (infinite, so that no cell passes, where they leave FP32's comfortable range)
   k.bound_c2 = (float)(p.gamma0 * (p.gamma0 - 1.0));
-  k.bound_floor = (float)(std::max(k.s.smallc2, p.gamma0 * p.smallp) * 1.001);
+  // and its floor takes in an energy that underflows in FP32, by 2^-149 before the
+  // division by the density and 2^-125 after it
+  k.bound_floor = (float)(std::max(k.s.smallc2, p.gamma0 * p.smallp) * 1.001 +
+                          p.gamma0 * (p.gamma0 - 1.0) *
+                              (std::ldexp(1.0, -148) / p.smallr + std::ldexp(1.0, -124)));
   const double lo = std::ldexp(1.0, -60), hi = std::ldexp(1.0, 60);
   const bool fits = p.dx > lo && p.dx < hi && p.dy > lo && p.dy < hi;
   k.bound_idx = fits ? (float)(1.00002 / p.dx) : HUGE_VALF;
