@@ -113,12 +113,15 @@ using Q4 = Q4T<double>;
 // Bounded kinds (BND).  Where the floors of the deck are not absurdly small
 // (SchemeT::floor_sqrt, decided on the host) most of those tests follow from
 // ranges that are cheap to check once per cell:
-//   d <= 2^40, p <= 2^90, (u^2 + v^2) / 2 <= 2^100, and the residuals of the
-//   quotients u, v and E / d zero or normal.
-// Then smallr >= 2^-60 <= d makes d and 1/d normal; a normal residual means a
-// numerator of at least 2^-970, so u, v and E / d are zero or at least 2^-1010,
-// and their differences zero or at least 2^-1062; p >= smallr smallp >= 2^-182
-// makes pressure differences zero or at least 2^-235.  With dt / dx <= 2^40
+//   d <= 2^40, p <= 2^90, (u^2 + v^2) / 2 <= 2^100, momenta zero or at least
+//   2^-901, and the residual of E / d zero or normal.
+// Then smallr >= 2^-60 <= d makes d and 1/d normal, and with a residual, a multiple
+// of 2^-106 of its numerator, zero or normal the quotients are the IEEE ones.  u and
+// v are zero or at least 2^-942 and their differences zero or at least 2^-995, so
+// that their halves are exact (a zero residual alone would not bound them: over
+// d = 1 every denormal divides exactly).  E / d enters the pressure only;
+// p >= smallr smallp >= 2^-182 makes pressure differences zero or at least 2^-235.
+// With dt / dx <= 2^40
 // (checked per wavefront) the traced face states stay below 2^190 in density,
 // pressure and velocity, far from overflow in every product of the solvers.
 // A wavefront with a lane outside these ranges takes the IEEE divisions.
@@ -142,6 +145,7 @@ constexpr int kClassZeroOrNormal = kClassNormal | (1 << 5) | (1 << 6);
 
 constexpr double kBndDensity = 0x1p40, kBndPressure = 0x1p90, kBndKinetic = 0x1p100;
 constexpr double kBndDtd = 0x1p40;  // dt / dx, dt / dy
+constexpr int kBndMomentumExp = -900;  // frexp exponent: zero (exponent 0) or >= 2^-901
 
 // a / d from r = 1 / d where no step needs scaling and a is not -0
 __device__ __forceinline__ double quot_plain(double a, double d, double r) {
@@ -202,8 +206,10 @@ __device__ __forceinline__ bool out_of_bounds(const Q4T<double> &q) {
 // reciprocal and no fallback.  Returns whether this lane's quotients are the
 // IEEE ones (BND: and the cell is in the bounded ranges); r is the reciprocal
 // and rok whether other quotients by d formed from it can be (d and r normal;
-// BND: part of the result instead).
-template <bool BND = false>
+// BND: part of the result instead).  RATE: for the CFL rate, where the sound speed
+// covers velocities whose quotients are too small to be exact, so that the momenta
+// are not tested (large ones and NaN fail the kinetic energy's bound).
+template <bool BND = false, bool RATE = false>
 __device__ __forceinline__ bool prim_fp64_shared(const SchemeT<double> &s, double u0, double u1,
                                                  double u2, double u3, Q4T<double> &q, double &r,
                                                  bool &rok) {
@@ -212,8 +218,11 @@ __device__ __forceinline__ bool prim_fp64_shared(const SchemeT<double> &s, doubl
   if constexpr (BND) {
     rok = true;
     bool ok = d <= kBndDensity;
-    const double ux = __builtin_copysign(quot_resid(u2, d, r, ok), u2);  // d > 0
-    const double uy = __builtin_copysign(quot_resid(u3, d, r, ok), u3);
+    if constexpr (!RATE)
+      ok = ok && min(__builtin_amdgcn_frexp_exp(u2), __builtin_amdgcn_frexp_exp(u3)) >=
+                     kBndMomentumExp;
+    const double ux = __builtin_copysign(quot_plain(u2, d, r), u2);  // d > 0
+    const double uy = __builtin_copysign(quot_plain(u3, d, r), u3);
     const double e1 = quot_resid(u1, d, r, ok);
     const double eken = prim_finish(s, d, ux, uy, e1, q);
     return ok && q.v[IP] <= kBndPressure && eken <= kBndKinetic;
@@ -335,7 +344,7 @@ __device__ __forceinline__ double cfl_rate_fp64(const Scheme &s, double u0, doub
   Q4 q;
   double r;
   bool rok;
-  bool ok = prim_fp64_shared<FS>(s, u0, u1, u2, u3, q, r, rok);
+  bool ok = prim_fp64_shared<FS, FS>(s, u0, u1, u2, u3, q, r, rok);
   // bounded: smallp <= p / d <= 2^150, nothing to scale
   double x = FS ? quot_plain(s.gamma0 * q.v[IP], q.v[ID], r)
                 : quot_shared(s.gamma0 * q.v[IP], q.v[ID], r, rok);
