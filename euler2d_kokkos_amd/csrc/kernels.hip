@@ -2274,11 +2274,16 @@ KParams make_kparams(const e2d_params &p, int precision) {
   // rate_below's constants: the last factor of its margin is in the cell sizes
   // (infinite, so that no cell passes, where they leave FP32's comfortable range)
   k.bound_c2 = (float)(p.gamma0 * (p.gamma0 - 1.0));
-  // and its floor takes in an energy that underflows in FP32, by 2^-149 before the
-  // division by the density and 2^-125 after it
+  // and its floor takes in what FP32's smallest number, 2^-149, rounds off: before the
+  // division by the density (at least smallr) up to 2^-150 of an energy or a momentum,
+  // after it 2^-150 of their quotients.  Energies for which that is more than 2^-20 of
+  // the whole, and velocities for which it is more than 2^-17 of the sound speed, lie
+  // below the floor; 2^-120 keeps the bound itself a normal number.
+  const double lost = std::ldexp(1.0, -150) / p.smallr + std::ldexp(1.0, -150);
+  const double lost_v = lost * std::ldexp(1.0, 17);
   k.bound_floor = (float)(std::max(k.s.smallc2, p.gamma0 * p.smallp) * 1.001 +
-                          p.gamma0 * (p.gamma0 - 1.0) *
-                              (std::ldexp(1.0, -148) / p.smallr + std::ldexp(1.0, -124)));
+                          p.gamma0 * (p.gamma0 - 1.0) * lost * std::ldexp(1.0, 20) +
+                          lost_v * lost_v + std::ldexp(1.0, -120));
   const double lo = std::ldexp(1.0, -60), hi = std::ldexp(1.0, 60);
   const bool fits = p.dx > lo && p.dx < hi && p.dy > lo && p.dy < hi;
   k.bound_idx = fits ? (float)(1.00002 / p.dx) : HUGE_VALF;

@@ -101,3 +101,17 @@ def test_largest_rate_of_a_field(gpu_available, nx, slope):
     rho = np.where((pick > 0.2) & (pick < 0.21), p.smallr, rho)
     a = np.stack((rho, e * rho + 0.5 * rho * (u * u + v * v), rho * u, rho * v), axis=-1)
     _compare(p, a, f"field {nx} slope {slope}")
+
+
+@pytest.mark.parametrize("riemann", [1, 2], ids=["hll", "hllc"])
+@pytest.mark.parametrize("units", [3.49, 8.499, 100.499])
+def test_largest_rate_of_partly_lost_energies(gpu_available, units, riemann):
+    """Energies of a few units of FP32's smallest number, which the bound's conversion
+    rounds down, at the density floor.  The lower part has the same pressure, and a
+    density that puts its rate between the upper part's and the one that the rounded
+    energy would give."""
+    p = _params(riemannSolverType=riemann, smallr=FLOOR, smallc=FLOOR)
+    e = units * 2.0**-149
+    lower = 0.5 * (units + np.floor(units)) / units  # its squared rate over the upper part's
+    a = _uniform(p, (FLOOR / lower, e, 0.0), (FLOOR, e, 0.0))
+    _compare(p, a, f"{units} units riemann {riemann}")
