@@ -670,6 +670,13 @@ int create_run(const e2d_params *p, int precision, char *arrays, e2d_run **out) 
     int ncu = 0;
     HIP_TRY(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, r->device));
     r->kp.simds = 4 * ncu;
+    // 32-bit row offsets in the step kernels need planes of at most 4 GiB;
+    // E2D_WIDE_ADDRESSING=1 selects the 64-bit form for any size
+    const char *wide = std::getenv("E2D_WIDE_ADDRESSING");
+    r->kp.wide_addr = (wide && *wide && std::strcmp(wide, "0") != 0) ||
+                      (unsigned long long)grid_shape(r->p, precision).plane *
+                              e2d::grid_scalar_bytes(precision) >
+                          (1ull << 32);
     r->seg_rows = e2d::auto_tile(r->kp);
     HIP_TRY(hipStreamCreateWithFlags(&r->stream, hipStreamNonBlocking));
     void *ptr = nullptr;
@@ -700,12 +707,6 @@ int create_run(const e2d_params *p, int precision, char *arrays, e2d_run **out) 
                           hipHostMallocDefault));
     std::memset(r->host_s, 0, host_bytes);
     r->host_rate = reinterpret_cast<double *>(r->host_s + 3);
-    // 32-bit row offsets in the step kernels need planes of at most 4 GiB;
-    // E2D_WIDE_ADDRESSING=1 selects the 64-bit form for any size
-    const char *wide = std::getenv("E2D_WIDE_ADDRESSING");
-    r->kp.wide_addr = (wide && *wide && std::strcmp(wide, "0") != 0) ||
-                      (unsigned long long)r->U.plane * e2d::grid_scalar_bytes(precision) >
-                          (1ull << 32);
     // defined contents everywhere (ghosts included) before the first init
     const size_t bytes = grid_bytes(r->U, precision);
     HIP_TRY(hipMemsetAsync(r->U.p, 0, bytes, r->stream));

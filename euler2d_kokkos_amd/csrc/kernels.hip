@@ -2443,7 +2443,7 @@ hipError_t launch_step_fused(const KParams &kp, Grid in, Grid out, double dt, St
 
 BlockMap block_map(const KParams &kp, int seg_rows) {
   BlockMap m{};
-  if (seg_rows > 2 * block_max_waves(2) - 4) return m;
+  if (seg_rows > 2 * block_max_waves(2) - 4 || kp.wide_addr) return m;
   // built for HLL and HLLC, in FP64 for the bounded kinds
   if (kp.s.riemann == 0 || (kp.prec == E2D_PRECISION_FP64 && !kp.s.floor_sqrt)) return m;
   const int k = seg_rows <= block_max_waves(1) - 4 ? 1 : 2;

@@ -163,7 +163,8 @@ struct BlockMap {
 };
 // wavefronts of the largest block: as many as a CU holds at the kernel's registers
 constexpr int block_max_waves(int k) { return k == 1 ? 16 : 12; }
-// A tile runs the block kernel where its blocks fit one per CU of the device.
+// A tile runs the block kernel where its blocks fit one per CU of the device (with
+// 32-bit row offsets: not where kp.wide_addr is set).
 BlockMap block_map(const KParams &kp, int seg_rows);
 
 // Relative time of a step whose `waves` wavefronts march `tile` rows each (plus
