@@ -2230,8 +2230,9 @@ KParams make_kparams(const e2d_params &p, int precision) {
   k.s.smallc2 = p.smallc * p.smallc;
   // the short square root for the wave speeds (arguments >= smallc^2) and the
   // CFL rate, and the floors from which the bounded quotients' ranges follow
-  k.s.floor_sqrt = p.smallr >= std::ldexp(1.0, -60) && p.smallc >= std::ldexp(1.0, -60) &&
-                           p.smallr * p.smallp >= std::ldexp(1.0, -182) &&
+  k.s.floor_sqrt = p.smallr >= std::ldexp(1.0, -110) && p.smallc >= std::ldexp(1.0, -110) &&
+                           p.smallc <= std::ldexp(1.0, 200) &&
+                           p.smallp >= std::ldexp(1.0, -230) &&
                            p.gamma0 <= 16.0 && k.s.entho <= std::ldexp(1.0, 20) &&
                            p.dx >= std::ldexp(1.0, -100) && p.dx <= std::ldexp(1.0, 100) &&
                            p.dy >= std::ldexp(1.0, -100) && p.dy <= std::ldexp(1.0, 100)

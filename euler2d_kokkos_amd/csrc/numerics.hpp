@@ -45,7 +45,7 @@ struct Ops<double> {
 // x itself for +-0 and +inf.  For x in [2^-767, DBL_MAX] the scaling and the
 // special cases are identities, so the same core sequence, operation for
 // operation, gives the same bits; the host enables it only when smallc^2 (the
-// floor of every argument) is >= 2^-120.  +inf gives NaN where sqrt returns inf.
+// floor of every argument) is >= 2^-220.  +inf gives NaN where sqrt returns inf.
 __device__ __forceinline__ double sqrt_core(double x) {
   const double y = __builtin_amdgcn_rsq(x);
   double g = x * y;
@@ -82,8 +82,8 @@ struct SchemeT {
   T gamma0, gamma6, smallr, smallc, smallp, smallpp, slope_type, entho;
   T smallc2;    // smallc * smallc
   int riemann;  // 0 approx, 1 hll, 2 hllc (already resolved from honor_riemann)
-  // smallr and smallc >= 2^-60, smallr*smallp >= 2^-182, gamma0 <= 16, entho <= 2^20, cell
-  // sizes of 2^-100 .. 2^100: the sound speeds take the short sqrt and the step's
+  // smallr >= 2^-110, smallc 2^-110 .. 2^200, smallp >= 2^-230, gamma0 <= 16, entho <= 2^20,
+  // cell sizes of 2^-100 .. 2^100: the sound speeds take the short sqrt and the step's
   // quotients the bounded forms
   int floor_sqrt;
 };
@@ -113,18 +113,25 @@ using Q4 = Q4T<double>;
 // Bounded kinds (BND).  Where the floors of the deck are not absurdly small
 // (SchemeT::floor_sqrt, decided on the host) most of those tests follow from
 // ranges that are cheap to check once per cell:
-//   d <= 2^40, p <= 2^90, (u^2 + v^2) / 2 <= 2^100, momenta zero or at least
-//   2^-901, and the residual of E / d zero or normal.
-// Then smallr >= 2^-60 <= d makes d and 1/d normal, and with a residual, a multiple
+//   d <= 2^80, p <= 2^160, (u^2 + v^2) / 2 <= 2^120, momenta zero or at least
+//   2^-801, and the residual of E / d zero or normal.
+// Then smallr >= 2^-110 <= d makes d and 1/d normal, and with a residual, a multiple
 // of 2^-106 of its numerator, zero or normal the quotients are the IEEE ones.  u and
-// v are zero or at least 2^-942 and their differences zero or at least 2^-995, so
+// v are zero or at least 2^-881 and their differences zero or at least 2^-934, so
 // that their halves are exact (a zero residual alone would not bound them: over
 // d = 1 every denormal divides exactly).  E / d enters the pressure only;
-// p >= smallr smallp >= 2^-182 makes pressure differences zero or at least 2^-235.
-// With dt / dx <= 2^40
-// (checked per wavefront) the traced face states stay below 2^190 in density,
-// pressure and velocity, far from overflow in every product of the solvers.
-// A wavefront with a lane outside these ranges takes the IEEE divisions.
+// p >= smallr smallp >= 2^-340 makes pressure differences zero or at least 2^-393.
+// With dt / dx <= 2^40 (checked per wavefront) the traced face states stay below
+// 2^185 in density, 2^268 in pressure (2^455 once floored, for a large smallp) and
+// 2^311 in velocity, and the wave speeds below 2^200; what may still overflow in the
+// solvers is named there.  A wavefront with a lane outside these ranges takes the
+// IEEE divisions, for a cell out of them in all of its later rows, after the checked
+// forms: 1024x1536, 14 rows, 71 us with every wavefront outside, 42.5 with none; 55 with
+// a disc of 0.1% of the cells outside.  Floors below the ranges leave the deck to the
+// kinds with IEEE divisions: 49.6 us.  The ranges keep both to values that no system
+// of units brings about (1e24 in density, 1e48 in pressure, 1e18 in velocity; floors
+// under 1e-33).  A branch around the checked forms for wavefronts outside costs all
+// others more than it saves: 42.5 -> 43.8 us, 768x384 17.1 -> 19.0.
 //
 // The march is bound by VALU issue (4 cycles per FP64 instruction, 16 per rcp
 // or rsq), so these forms, one wave-speed root per face instead of two, the
@@ -143,9 +150,9 @@ __device__ __forceinline__ double recip_newton(double d) {
 constexpr int kClassNormal = (1 << 3) | (1 << 8);
 constexpr int kClassZeroOrNormal = kClassNormal | (1 << 5) | (1 << 6);
 
-constexpr double kBndDensity = 0x1p40, kBndPressure = 0x1p90, kBndKinetic = 0x1p100;
+constexpr double kBndDensity = 0x1p80, kBndPressure = 0x1p160, kBndKinetic = 0x1p120;
 constexpr double kBndDtd = 0x1p40;  // dt / dx, dt / dy
-constexpr int kBndMomentumExp = -900;  // frexp exponent: zero (exponent 0) or >= 2^-901
+constexpr int kBndMomentumExp = -800;  // frexp exponent: zero (exponent 0) or >= 2^-801
 
 // a / d from r = 1 / d where no step needs scaling and a is not -0
 __device__ __forceinline__ double quot_plain(double a, double d, double r) {
@@ -319,8 +326,8 @@ __device__ __forceinline__ T cfl_rate_q(const SchemeT<T> &s, const Q4T<T> &q, co
 
 // The rate's square root of gamma p / d.  p >= d smallp, and under the host's
 // floor_sqrt condition (which keeps d smallp normal for every d >= smallr) the
-// argument is at least smallc^2 (1 - 5u) > 2^-121, where the short sequence gives
-// the IEEE bits; +inf keeps sqrt's result, and NaN stays NaN.
+// argument is at least smallp > 2^-231, where the short sequence gives the IEEE
+// bits; +inf keeps sqrt's result, and NaN stays NaN.
 template <bool FS>
 __device__ __forceinline__ double rate_sqrt(double x) {
   if constexpr (FS) {
@@ -345,7 +352,7 @@ __device__ __forceinline__ double cfl_rate_fp64(const Scheme &s, double u0, doub
   double r;
   bool rok;
   bool ok = prim_fp64_shared<FS, FS>(s, u0, u1, u2, u3, q, r, rok);
-  // bounded: smallp <= p / d <= 2^150, nothing to scale
+  // bounded: 2^-230 <= smallp <= p / d <= 2^270, nothing to scale
   double x = FS ? quot_plain(s.gamma0 * q.v[IP], q.v[ID], r)
                 : quot_shared(s.gamma0 * q.v[IP], q.v[ID], r, rok);
   const bool all = wave_all(ok && rok);
@@ -360,7 +367,7 @@ __device__ __forceinline__ double cfl_rate_fp64(const Scheme &s, double u0, doub
   if constexpr (FS) {
     // The cell sizes' correctly rounded reciprocals are at hand: with them the
     // residual step gives the IEEE quotient (Markstein 1990) wherever nothing
-    // leaves the normal range (speeds of 2^-62 .. 2^52 here, cell sizes of 2^-100 ..
+    // leaves the normal range (speeds of 2^-116 .. 2^138 here, cell sizes of 2^-100 ..
     // 2^100 by the host's floor_sqrt condition).  3 instructions instead of 11, one
     // of them a reciprocal, per direction.
     double rx = quot_plain(vx, rt.dx, rt.idx), ry = quot_plain(vy, rt.dy, rt.idy);
@@ -563,11 +570,14 @@ __device__ __forceinline__ T wave_speed(const SchemeT<T> &s, T pl, T rl, T pr, T
 // BND: the two quotients by rcr + rcl share a reciprocal, as do the two by
 // Sk - ustar; ok is cleared in a lane where one of them may differ from the
 // IEEE quotient.  Of the bounded ranges' consequences these are left to test:
-// rcr + rcl (2^-150 .. 2^40) and Sk - ustar away from zero, and the residuals of ustar and
-// etotstar, whose numerators may be tiny (those of ptotstar and rstar are
-// zero or at least 2^-410; an overflow anywhere makes the last residual NaN
-// or infinite).  No numerator is ever -0: each ends in a sum with +0 or with a
-// number that is not zero.
+// rcr + rcl (2^-230 .. 2^301) and Sk - ustar (2^-200 at least), and the residuals of
+// ustar and etotstar, whose numerators may be tiny.  rcl and rcr are zero or at least
+// smallr smallc / 2 >= 2^-221, as is rstar's numerator, and ptotstar's is zero or at
+// least 2^-615 (the rounding of its positive part, 2^-221 2^-340).  ustar stays
+// below 2^686 and rstar between 2^-907 and 2^698, or zero.  An overflow on the way to
+// ustar or ptotstar makes etotstar's numerator, and with it the last residual, NaN
+// or infinite.  No numerator is ever -0: each ends in a sum with +0 or with a number
+// that is not zero.
 template <bool FS = false, bool BND = false, class T>
 __device__ __forceinline__ void hllc(const SchemeT<T> &s, const Q4T<T> &ql, const Q4T<T> &qr,
                                      int ln, int tn, T flux[4], bool &ok) {
@@ -595,7 +605,7 @@ __device__ __forceinline__ void hllc(const SchemeT<T> &s, const Q4T<T> &ql, cons
   T ustar, ptotstar;
   if constexpr (BND) {
     const T r = recip_newton(rc);
-    ok = ok && exponent_within(rc, -150, 40);
+    ok = ok && exponent_within(rc, -230, 300);
     ustar = quot_resid(un, rc, r, ok);
     ptotstar = quot_plain(pn, rc, r);
   } else {
@@ -648,8 +658,8 @@ __device__ __forceinline__ void hllc(const SchemeT<T> &s, const Q4T<T> &ql, cons
 // HLL (no reference counterpart; the reference declares the enum only,
 // HydroParams.h:49).  Toro 2009, section 10.3, eq. (10.21), with the floors and
 // wave speeds of riemann_hllc.  Same expressions as the CPU oracle.  BND: SR - SL
-// is at least 2^-113 wherever the middle state is taken, so its reciprocal needs
-// no test.
+// is at least smallc wherever the middle state is taken, and below 2^313, so its
+// reciprocal needs no test.
 template <bool FS = false, bool BND = false, class T>
 __device__ __forceinline__ void hll(const SchemeT<T> &s, const Q4T<T> &ql, const Q4T<T> &qr,
                                     int ln, int tn, T flux[4]) {
