@@ -971,34 +971,6 @@ enum : int {
 // 16384x8192 grids, and the split step 3-8% faster at tiles of 20 rows or
 // more, but 4% slower at its best tile of 14 rows (launch_fused_t).
 
-// The CFL rate of a step is the maximum over its cells, and the exact FP64 rate
-// of a cell costs a reciprocal, a square root and 90 instructions in all.  This
-// test costs 28, most of them FP32: a bound from above on the cell's rate, below a
-// rate already found.  The conversion's rounding errors are within 2^-21
-// (|E| / d + v^2) in the specific internal energy, which the 2^-19 term covers,
-// and within 2^-20 relative in everything else, which the factor in the inverse
-// cell sizes covers; what underflows in FP32 is covered by bound_floor.  Densities
-// whose reciprocal could underflow, speeds above 2^50 (whose square could leave
-// FP32's range and take the sound speed out of the bound) and energies past FP32's
-// range are never below.  Cells that pass cannot exceed a rate that takes part in
-// the maximum, so the maximum keeps its bits.
-__device__ __forceinline__ bool rate_below(const KParams &kp, const double u[4], float found) {
-  const float d = fmaxf((float)u[0], kp.sf.smallr);
-  const float r = __builtin_amdgcn_rcpf(d);
-  const float vx = (float)u[2] * r, vy = (float)u[3] * r, e1 = (float)u[1] * r;
-  const float k = __builtin_fmaf(vx, vx, vy * vy);
-  const float e = __builtin_fmaf(-0.5f, k, e1);
-  const float em = __builtin_fmaf(fabsf(e1) + k, 0x1p-19f, e);
-  const float c = __builtin_amdgcn_sqrtf(fmaxf(kp.bound_c2 * em, kp.bound_floor));
-  const float bound = __builtin_fmaf(c + fabsf(vx), kp.bound_idx, (c + fabsf(vy)) * kp.bound_idy);
-  return bound < found && d <= 0x1p100f && k <= 0x1p100f;
-}
-
-// a finite float below the rate
-__device__ __forceinline__ float rate_found(double rate) {
-  return fminf((float)rate * (1.0f - 0x1p-22f), __FLT_MAX__);
-}
-
 // Everything one wavefront carries while marching up its strip.
 template <class P>
 struct MarchState {
@@ -1012,7 +984,6 @@ struct MarchState {
   // bounded FP64 kinds, wave-uniform: rows r-1 and r-2 passed the conversion's
   // check; a cell outside the bounded ranges was met (or dt / dx is)
   bool ok1, ok2, slow;
-  float found;  // kPruneRate: below some rate of this step found by now (wave-uniform)
 };
 
 // One iteration over loaded row r.  STAGES is a compile-time set, so the
@@ -1178,17 +1149,16 @@ __device__ __forceinline__ void march_row(const KParams &kp, const Grid &in, con
     const int b = r - 2;
     const bool mine = out_col && (!ROWS || b <= kp.ny + 1);
     if (mine) P::template store_rc<O32>(out, b, pin_offset((unsigned)col * P::kElem), unew);
-    if constexpr (RATE) {  // next-step CFL rate of the new state
+    if constexpr (RATE) {
+      // Next-step CFL rate of the new state, of every cell.  Leaving out a row's exact
+      // rate where an FP32 bound lies below a rate already found (28 instructions
+      // for 90) needs a branch, which splits the row.  8192x8192 HLL, every cell / with
+      // the bound: four quadrants 1257 / 1300 us, uniform 1309 / 1458, blast 1318 / 1352; only
+      // states without a uniform part of the largest rate gain (implode 1310 / 1278).
+      // Giving the bound up after eight rows that it does not cover: 1264, 1391, 1332,
+      // 1290; a loop with and one without it, chosen by the first row: slower than both.
       constexpr bool kFs = (RS & kRiemannFloorSqrt) != 0, kPow2 = (RS & kMinmodPow2) != 0;
-      if constexpr ((RS & kPruneRate) != 0) {
-        // only where some cell may exceed the rate already found
-        if (!wave_all(!mine || rate_below(kp, unew.u, m.found))) {  // uniform
-          if (mine) m.wmax = fmax(m.wmax, cell_rate<P, kFs, kPow2>(kp, unew));
-          m.found = fmaxf(m.found, rate_found(wave_max(m.wmax)));
-        }
-      } else if (mine) {
-        m.wmax = Ops<T>::mx(m.wmax, cell_rate<P, kFs, kPow2>(kp, unew));
-      }
+      if (mine) m.wmax = Ops<T>::mx(m.wmax, cell_rate<P, kFs, kPow2>(kp, unew));
     }
   }
   if constexpr ((STAGES & kYFace) != 0) {
@@ -1230,7 +1200,7 @@ __device__ __forceinline__ void set_prio_level(int lvl) {
 template <int RS, class P, bool RATE, bool O32, bool COLS, int PD, class Start>
 __device__ __forceinline__ typename P::T march(const KParams &kp, const Grid &in, const Grid &out,
                                                Start &&start, int seg_rows, int nstrips,
-                                               int strip, int seg, bool prio, float found) {
+                                               int strip, int seg, bool prio) {
   using T = typename P::T;
   const int lane = threadIdx.x & (kLanes - 1);
 
@@ -1286,7 +1256,6 @@ __device__ __forceinline__ typename P::T march(const KParams &kp, const Grid &in
   m.ok1 = m.ok2 = true;
   m.slow = !wave_all((double)dtdx <= kBndDtd && (double)dtdy <= kBndDtd);
   m.wmax = T(0.0);
-  m.found = found;
 
   const int r0 = j_base - 2;
   // rows this segment updates: seg_rows, fewer in a top segment that ends at
@@ -1477,14 +1446,6 @@ void step_fused_kernel(KParams kp, Grid in, Grid out,
     }
     return go;
   };
-  float found = 0.0f;
-  if constexpr ((RS & kPruneRate) != 0) {  // start from the rates that earlier wavefronts found
-    const int lane = threadIdx.x & (kLanes - 1), p1 = ph == 2 ? 0 : ph + 1;
-    const unsigned long long b =
-        __hip_atomic_load(&ctl->rate[p1][(lane % kRateSlots) * kSlotStride], __ATOMIC_RELAXED,
-                          __HIP_MEMORY_SCOPE_AGENT);
-    found = rate_found(lane_value(row_max(__longlong_as_double((long long)b)), 0));
-  }
   int strip, seg, tile;
   fused_wave(fm, wave, strip, seg, tile);
   // in and out share their geometry (checked at launch): one pitch and one
@@ -1494,10 +1455,10 @@ void step_fused_kernel(KParams kp, Grid in, Grid out,
   T wmax;
   if (interior_cols(kp, strip))  // uniform
     wmax = march<RS, P, LOOP, O32, false, PD>(kp, in, o, start, tile, fm.nstrips, strip, seg,
-                                              fm.prio != 0, found);
+                                              fm.prio != 0);
   else
     wmax = march<RS, P, LOOP, O32, true, PD>(kp, in, o, start, tile, fm.nstrips, strip, seg,
-                                             fm.prio != 0, found);
+                                             fm.prio != 0);
   // run loop: the CFL rate of the step's output, for the next launch's dt
   if constexpr (LOOP) {
     if (go) reduce_rate_wave(wmax, rate_slot(ctl, ph));
@@ -1753,12 +1714,10 @@ __device__ __forceinline__ void batch_step_wave(const BatchInst *__restrict__ in
   T wmax;
   if (interior_cols(kp, it.strip))
     wmax = march<RS, P, true, O32, false, kBatchPrefetch<P>>(kp, gin, gout, start, it.rows,
-                                                             bi.nstrips, it.strip, it.seg, prio,
-                                                             0.0f);
+                                                             bi.nstrips, it.strip, it.seg, prio);
   else
     wmax = march<RS, P, true, O32, true, kBatchPrefetch<P>>(kp, gin, gout, start, it.rows,
-                                                            bi.nstrips, it.strip, it.seg, prio,
-                                                            0.0f);
+                                                            bi.nstrips, it.strip, it.seg, prio);
   if (go) reduce_rate_wave(wmax, rate_slot(ctl, ph));
 }
 
@@ -1931,10 +1890,10 @@ __device__ __forceinline__ void batch_persistent_loop(const BatchInst *__restric
       };
       if (interior_cols(kp, strip))
         wmax = march<RS, P, true, O32, false, kBatchPrefetch<P>>(kp, gin, gout, start, seg_rows, bi.nstrips,
-                                                 strip, seg, false, 0.0f);
+                                                 strip, seg, false);
       else
         wmax = march<RS, P, true, O32, true, kBatchPrefetch<P>>(kp, gin, gout, start, seg_rows, bi.nstrips,
-                                                strip, seg, false, 0.0f);
+                                                strip, seg, false);
       reduce_rate_wave(wmax, rate_slot(ctl, ph));
     }
     // this wavefront's stores and atomics are complete before it counts
@@ -2088,15 +2047,6 @@ void launch_fused_t(const KParams &kp, Grid in, Grid out, double dt, StepCtl *ct
   // the FP32 paths from 20-row tiles on
   const bool pd2 = seg_rows >= (std::is_same<P, P64>::value ? 8 : 20);
   if (ctl && off32_ok(kp, in) && off32_ok(kp, out)) {
-    if constexpr (std::is_same<P, P64>::value && (RS & kRiemannFloorSqrt) != 0) {
-      // more than two rounds of wavefronts: cells that cannot hold the largest
-      // rate are skipped (kPruneRate)
-      if (pd2 && kp.simds > 0 && fm.nwaves > 4 * kp.simds) {
-        hipLaunchKernelGGL((step_fused_kernel<RS | kPruneRate, P, true, true, 2>), dim3(blocks),
-                           dim3(kBlock), 0, st, kp, in, out, dt, ctl, ph, fm);
-        return;
-      }
-    }
     if (pd2)
       hipLaunchKernelGGL((step_fused_kernel<RS, P, true, true, 2>), dim3(blocks), dim3(kBlock), 0,
                          st, kp, in, out, dt, ctl, ph, fm);
@@ -2272,23 +2222,6 @@ KParams make_kparams(const e2d_params &p, int precision) {
     int e = 0;
     return h > 0.0 && std::frexp(h, &e) == 0.5 && e > -125 && e < 126;
   };
-  // rate_below's constants: the last factor of its margin is in the cell sizes
-  // (infinite, so that no cell passes, where they leave FP32's comfortable range)
-  k.bound_c2 = (float)(p.gamma0 * (p.gamma0 - 1.0));
-  // and its floor takes in what FP32's smallest number, 2^-149, rounds off: before the
-  // division by the density (at least smallr) up to 2^-150 of an energy or a momentum,
-  // after it 2^-150 of their quotients.  Energies for which that is more than 2^-20 of
-  // the whole, and velocities for which it is more than 2^-17 of the sound speed, lie
-  // below the floor; 2^-120 keeps the bound itself a normal number.
-  const double lost = std::ldexp(1.0, -150) / p.smallr + std::ldexp(1.0, -150);
-  const double lost_v = lost * std::ldexp(1.0, 17);
-  k.bound_floor = (float)(std::max(k.s.smallc2, p.gamma0 * p.smallp) * 1.001 +
-                          p.gamma0 * (p.gamma0 - 1.0) * lost * std::ldexp(1.0, 20) +
-                          lost_v * lost_v + std::ldexp(1.0, -120));
-  const double lo = std::ldexp(1.0, -60), hi = std::ldexp(1.0, 60);
-  const bool fits = p.dx > lo && p.dx < hi && p.dy > lo && p.dy < hi;
-  k.bound_idx = fits ? (float)(1.00002 / p.dx) : HUGE_VALF;
-  k.bound_idy = fits ? (float)(1.00002 / p.dy) : HUGE_VALF;
   k.rd = RateT<double>{p.dx, p.dy, 1.0 / p.dx, 1.0 / p.dy, pow2(p.dx), pow2(p.dy)};
   k.rf = RateT<float>{k.dxf, k.dyf, (float)(1.0 / p.dx), (float)(1.0 / p.dy), pow2(p.dx),
                       pow2(p.dy)};

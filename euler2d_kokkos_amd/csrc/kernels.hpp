@@ -35,7 +35,6 @@ struct KParams {
   float dxf, dyf;
   RateT<double> rd;     // cell sizes of the CFL rate (FP64 / FP32 arithmetic)
   RateT<float> rf;
-  float bound_c2, bound_floor, bound_idx, bound_idy;  // rate_below()
   // split path: primitive conversion redone in FP64 where the internal energy
   // is below this fraction of the total energy (p < kin_frac * (gamma-1) * E)
   float kin_frac;

@@ -792,13 +792,6 @@ constexpr int kMinmodPow2 = 16;
 // + kSlopeMinmod: the march's slopes alone are built for slope_type == 1 (any
 // cell sizes)
 constexpr int kSlopeMinmod = 32;
-// + kPruneRate: the march forms a cell's CFL rate only where it may exceed one
-// that the step has already found (bounded FP64 kinds, launches of more than two
-// rounds of wavefronts, whose later ones start from the rates found by then).
-// 8192x8192, 48-row tile: HLLC 1606 -> 1539 us, HLL 1544 -> 1487.  In a single round
-// each wavefront has to find its own first, and the test costs more than it
-// saves (1024x1536: 43.2 -> 46.2 us).
-constexpr int kPruneRate = 64;
 
 // BND: the states are in the bounded ranges; ok is cleared in a lane whose flux
 // may not have the IEEE bits

@@ -89,8 +89,8 @@ def test_states_at_the_floors(gpu_available, floors, thin, gamma, riemann, tile)
 @pytest.mark.parametrize("units", [3.49, 100.499])
 @pytest.mark.parametrize("gamma", [1 + 2.0**-20, 1.4])
 def test_largest_rate_at_the_lowest_floor(gpu_available, gamma, units):
-    """The rate bound where FP32 keeps an energy in part, as in test_gpu_rate, at the
-    lowest floor."""
+    """Rates of energies that FP32 would keep in part, as in test_gpu_rate, at the lowest
+    floor."""
     floor = 2.0**-110
     p = R._params(smallr=floor, smallc=floor, gamma0=gamma)
     lower = 0.5 * (units + np.floor(units)) / units

@@ -1,12 +1,12 @@
-"""The FP64 step that skips cells below a CFL rate already found.
+"""The largest CFL rate of a step, whatever the tile.
 
-Launches of more than two rounds of wavefronts (tiles of eight rows and more) form
-a cell's exact rate only where a bound in FP32 says that it may exceed one that
-the step has found; a tile of seven rows keeps every cell's rate.  The time step
-follows from the largest rate, so the times and the arrays of the two must agree
-bit for bit.  A cell whose rate the bound misses shows where the other cells'
-rates lie between the two: the grid's lower part holds those, in the wavefronts
-that march first, and its upper part the cell state in question.
+The time step follows from the largest rate of the step's output, which its wavefronts
+fold as they march; tiles of eight rows and of seven are different kernels (two rows
+loaded ahead, or one), and at these sizes eight rows are more than two rounds of
+wavefronts.  The times and the arrays of the two must agree bit for bit, also where the
+largest rate belongs to a few cells that a shorter or narrower evaluation would miss:
+the grid's lower part holds states of slightly smaller rate, in the wavefronts that
+march first, and its upper part the cell state in question.
 """
 import numpy as np
 import pytest
@@ -106,10 +106,9 @@ def test_largest_rate_of_a_field(gpu_available, nx, slope):
 @pytest.mark.parametrize("riemann", [1, 2], ids=["hll", "hllc"])
 @pytest.mark.parametrize("units", [3.49, 8.499, 100.499])
 def test_largest_rate_of_partly_lost_energies(gpu_available, units, riemann):
-    """Energies of a few units of FP32's smallest number, which the bound's conversion
-    rounds down, at the density floor.  The lower part has the same pressure, and a
-    density that puts its rate between the upper part's and the one that the rounded
-    energy would give."""
+    """Energies of a few units of FP32's smallest number, which FP32 would round down, at
+    the density floor.  The lower part has the same pressure, and a density that puts
+    its rate between the upper part's and the one that the rounded energy would give."""
     p = _params(riemannSolverType=riemann, smallr=FLOOR, smallc=FLOOR)
     e = units * 2.0**-149
     lower = 0.5 * (units + np.floor(units)) / units  # its squared rate over the upper part's
