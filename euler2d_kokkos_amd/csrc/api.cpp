@@ -13,8 +13,6 @@
 #include <cstring>
 #include <new>
 #include <string>
-#include <system_error>
-#include <thread>
 #include <utility>
 #include <vector>
 
@@ -26,6 +24,7 @@
 #include "params.hpp"
 #include "status.hpp"
 #include "trace.hpp"
+#include "workers.hpp"
 
 using e2d::Grid;
 
@@ -587,20 +586,7 @@ int stage_copy(const e2d_run *r, Staging &s, const Grid &g, double *host, int la
   };
 
   hipError_t err[kStageThreads] = {};
-  std::thread helpers[kStageThreads];
-  int mine = 1;  // chunk sequences 0 .. mine - 1 and those no thread could be started for
-  for (int t = 1; t < nthreads; ++t) {
-    try {
-      helpers[t] = std::thread([&, t] { err[t] = worker(t); });
-    } catch (const std::system_error &) {
-      break;
-    }
-    mine = t + 1;
-  }
-  err[0] = worker(0);
-  for (int t = mine; t < nthreads; ++t) err[t] = worker(t);
-  for (std::thread &h : helpers)
-    if (h.joinable()) h.join();
+  e2d::run_workers<kStageThreads>(nthreads, [&](int t) { err[t] = worker(t); });
   const hipError_t se = hipStreamSynchronize(r->stream);
   for (hipError_t e : err)
     if (e != hipSuccess) return hip_fail(e, "host copy");
