@@ -11,6 +11,7 @@
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
+#include <memory>
 #include <new>
 #include <string>
 #include <utility>
@@ -1284,7 +1285,6 @@ int batch_upload_queue(e2d_batch *b, const std::vector<int> &waves) {
     }
   }
   begin[nx] = (int)order.size();
-  b->queue_per_step = per;
   long long total = 0, most = 0;
   for (long long l : load) {
     total += l;
@@ -1299,6 +1299,7 @@ int batch_upload_queue(e2d_batch *b, const std::vector<int> &waves) {
   HIP_TRY(hipMemcpyAsync(b->queue_ints, h.data(), h.size() * sizeof(int), hipMemcpyHostToDevice,
                          b->stream));
   HIP_TRY(hipStreamSynchronize(b->stream));  // h is read before it goes
+  b->queue_per_step = std::move(per);
   b->queue.order = b->queue_ints;
   b->queue.wave_prefix = b->queue_ints + n;
   b->queue.xcd_begin = b->queue_ints + 2 * n;
@@ -1308,8 +1309,9 @@ int batch_upload_queue(e2d_batch *b, const std::vector<int> &waves) {
   return E2D_OK;
 }
 
-// instance table for the current tile
-int batch_upload_table(e2d_batch *b) {
+// The instance and item tables and the queues for a tile, which becomes the batch's
+// once they are in place: a refused allocation leaves the batch at its former tile.
+int batch_tile(e2d_batch *b, int seg_rows) {
   std::vector<e2d::BatchInst> h(b->runs.size());
   int waves = 0;
   long long cells = 0;
@@ -1322,51 +1324,52 @@ int batch_upload_table(e2d_batch *b) {
     bi.kp = r->kp;
     bi.U = r->U;
     bi.U2 = r->U2;
-    inst_waves[i] = e2d::batch_waves(r->kp, b->seg_rows, &bi.nstrips);
-    e2d::batch_items(r->kp, b->seg_rows, (int)i, items);
+    inst_waves[i] = e2d::batch_waves(r->kp, seg_rows, &bi.nstrips);
+    e2d::batch_items(r->kp, seg_rows, (int)i, items);
     waves += inst_waves[i];
     cells += (long long)r->p.nx * r->p.ny;
   }
-  b->nwaves = waves;
-  b->cells = cells;
   e2d::batch_order(h.data(), items);
-  batch_drop_graph(b);
+  struct DeviceFree {
+    void operator()(void *p) const { (void)hipFree(p); }
+  };
+  std::unique_ptr<void, DeviceFree> larger;
   if (items.size() > b->items_cap) {
-    HIP_TRY(hipStreamSynchronize(b->stream));
-    if (b->items) (void)hipFree(b->items);
-    b->items = nullptr;
-    b->items_cap = 0;
-    b->nitems = 0;
     void *ptr = nullptr;
-    if (hipMalloc(&ptr, items.size() * sizeof(e2d::BatchItem)) != hipSuccess)
+    if (hipMalloc(&ptr, items.size() * sizeof(e2d::BatchItem)) != hipSuccess) {
+      (void)hipGetLastError();
       return fail(E2D_ERR_ALLOC, "batch: device allocation failed");
-    b->items = static_cast<e2d::BatchItem *>(ptr);
+    }
+    larger.reset(ptr);
+  }
+  batch_drop_graph(b);
+  int rc = batch_upload_queue(b, inst_waves);  // waits for the stream
+  if (rc) return rc;
+  if (larger) {
+    if (b->items) (void)hipFree(b->items);
+    b->items = static_cast<e2d::BatchItem *>(larger.release());
     b->items_cap = items.size();
   }
   HIP_TRY(hipMemcpyAsync(b->items, items.data(), items.size() * sizeof(e2d::BatchItem),
                          hipMemcpyHostToDevice, b->stream));
-  b->nitems = (int)items.size();
   HIP_TRY(hipMemcpyAsync(b->insts, h.data(), h.size() * sizeof(e2d::BatchInst),
                          hipMemcpyHostToDevice, b->stream));
-  int rc = batch_upload_queue(b, inst_waves);
-  if (rc) return rc;
   HIP_TRY(hipStreamSynchronize(b->stream));
+  b->nitems = (int)items.size();
+  b->nwaves = waves;
+  b->cells = cells;
+  b->seg_rows = seg_rows;
   return E2D_OK;
 }
 
-int batch_tile(e2d_batch *b, int seg_rows) {
-  b->seg_rows = seg_rows;
-  return batch_upload_table(b);
-}
-
-// The tile of the current launch mode while the caller has chosen none.  One
+// The tile of a launch mode while the caller has chosen none.  One
 // launch per step: the march's least cost over all instances.  Persistent: no tail per
 // step, so FP64 takes longer segments, about 3.5 wavefronts per SIMD (192 instances,
 // tiles 14 / 32 / 64: 356 / 327 / 316 us), while split precision wants its third
 // wavefront per SIMD (prefetch distance 1, short segments; tiles 14 / 20 / 48: 229 /
 // 218 / 222 us).
-int batch_auto_tile(const e2d_batch *b) {
-  const bool persistent = b->launch == E2D_BATCH_LAUNCH_PERSISTENT;
+int batch_auto_tile(const e2d_batch *b, int mode) {
+  const bool persistent = mode == E2D_BATCH_LAUNCH_PERSISTENT;
   auto waves = [&](int tile) {
     long long w = 0;
     for (const e2d_run *r : b->runs)
@@ -1523,10 +1526,17 @@ int e2d_batch_set_launch(e2d_batch *b, int mode, int spin_limit) {
   if (rc) return rc;
   if (mode != E2D_BATCH_LAUNCH_STEPS && mode != E2D_BATCH_LAUNCH_PERSISTENT)
     return fail(E2D_ERR_ARG, "mode must be E2D_BATCH_LAUNCH_STEPS or _PERSISTENT");
+  if (!b->tile_chosen) {
+    rc = guarded([&]() -> int {
+      const int tile = batch_auto_tile(b, mode);
+      return tile == b->seg_rows ? E2D_OK : batch_tile(b, tile);
+    });
+    if (rc) return rc;
+  }
   b->launch = mode;
   b->launch_chosen = true;
   b->spin_limit = spin_limit > 0 ? (unsigned)spin_limit : 0u;
-  return guarded([&]() -> int { return b->tile_chosen ? E2D_OK : batch_tile(b, batch_auto_tile(b)); });
+  return E2D_OK;
 }
 
 int e2d_batch_get_launch(e2d_batch *b, int *mode) {
@@ -1644,7 +1654,7 @@ int e2d_batch_create(const e2d_params *params, int count, int precision, e2d_bat
       e2d_batch_destroy(b);
       return hip_fail(e, "hipMemsetAsync(batch tables)");
     }
-    int rc = batch_upload_table(b);
+    int rc = batch_tile(b, b->seg_rows);
     if (rc) {
       const std::string msg = g_last_error;
       e2d_batch_destroy(b);
@@ -1663,7 +1673,7 @@ int e2d_batch_create(const e2d_params *params, int count, int precision, e2d_bat
     b->launch = b->queue_imbalance <= kPersistentImbalance && count >= kPersistentPerQueue * b->nxcd
                     ? E2D_BATCH_LAUNCH_PERSISTENT
                     : E2D_BATCH_LAUNCH_STEPS;
-    rc = batch_tile(b, batch_auto_tile(b));
+    rc = batch_tile(b, batch_auto_tile(b, b->launch));
     if (rc) {
       const std::string msg = g_last_error;
       e2d_batch_destroy(b);
@@ -1718,8 +1728,9 @@ int e2d_batch_set_tile(e2d_batch *b, int seg_rows) {
   int rc = batch_check(b);
   if (rc) return rc;
   if (seg_rows < 1 || seg_rows > 4096) return fail(E2D_ERR_ARG, "seg_rows must be in [1, 4096]");
-  b->tile_chosen = true;
-  return guarded([&]() -> int { return batch_tile(b, seg_rows); });
+  rc = guarded([&]() -> int { return batch_tile(b, seg_rows); });
+  if (!rc) b->tile_chosen = true;
+  return rc;
 }
 
 int e2d_batch_run(e2d_batch *b, int max_steps, int use_graph, double *elapsed_ms,
