@@ -286,16 +286,6 @@ __device__ __forceinline__ void prim_no_c(const SchemeT<T> &s, T u0, T u1, T u2,
   }
 }
 
-// ComputeDtFunctor body, HydroRunFunctors.h:53-74: (c+|u|)/dx + (c+|v|)/dy
-template <class T>
-__device__ __forceinline__ T cfl_rate_q(const SchemeT<T> &s, const Q4T<T> &q, T dx, T dy) {
-  using O = Ops<T>;
-  const T c = O::sqroot(O::div(s.gamma0 * (q.v[IP]), q.v[ID]));
-  const T vx = c + O::ab(q.v[IU]);
-  const T vy = c + O::ab(q.v[IV]);
-  return O::div(vx, dx) + O::div(vy, dy);
-}
-
 // Cell sizes for the CFL rate.  When a cell size is an exact power of two its
 // reciprocal is exact and x / dx == x * (1/dx) for every x (IEEE division by
 // 2^-k is an exact scaling, overflow and NaN included), so the division is
@@ -306,6 +296,7 @@ struct RateT {
   int pow2x, pow2y;
 };
 
+// ComputeDtFunctor body, HydroRunFunctors.h:53-74: (c+|u|)/dx + (c+|v|)/dy
 template <class T>
 __device__ __forceinline__ T cfl_rate_q(const SchemeT<T> &s, const Q4T<T> &q, const RateT<T> &r) {
   using O = Ops<T>;
@@ -387,13 +378,6 @@ __device__ __forceinline__ double cfl_rate_fp64(const Scheme &s, double u0, doub
   else
     ry = vy / rt.dy;
   return rx + ry;
-}
-
-__device__ __forceinline__ double cfl_rate(const Scheme &s, double u0, double u1, double u2,
-                                           double u3, double dx, double dy) {
-  Q4 q;
-  prim_no_c(s, u0, u1, u2, u3, q);
-  return cfl_rate_q(s, q, dx, dy);
 }
 
 // neg ? -z : z as one select on the high word (with the operand's negation)
