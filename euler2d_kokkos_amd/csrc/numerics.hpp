@@ -527,9 +527,9 @@ __device__ __forceinline__ void trace_face(const SchemeT<T> &s, const Q4T<T> &q,
 // square root never decreases where its argument grows, so the root of the
 // larger argument is the larger root, bit for bit, and one root serves both
 // (the FP32 hardware root was checked to be monotone over every positive float).
-// FS: the short root, which gives NaN for +inf: its argument is capped at the
-// largest finite value.  BND: quotients of states in the bounded ranges.
-template <bool FS, bool BND, class T>
+// BND: states in the bounded ranges, whose quotients and root take the short forms
+// (the short root would give NaN for the +inf that other states may bring).
+template <bool BND, class T>
 __device__ __forceinline__ T wave_speed(const SchemeT<T> &s, T pl, T rl, T pr, T rr) {
   using O = Ops<T>;
   if constexpr (BND) {
@@ -538,7 +538,6 @@ __device__ __forceinline__ T wave_speed(const SchemeT<T> &s, T pl, T rl, T pr, T
     return sqrt_core(O::mx(O::mx(xl, xr), s.smallc2));
   } else {
     const T a = O::mx(O::mx(O::div(s.gamma0 * pl, rl), O::div(s.gamma0 * pr, rr)), s.smallc2);
-    if constexpr (FS) return sqrt_core(O::mn(a, T(__DBL_MAX__)));
     return O::sqroot(a);
   }
 }
@@ -562,7 +561,7 @@ __device__ __forceinline__ T wave_speed(const SchemeT<T> &s, T pl, T rl, T pr, T
 // ustar or ptotstar makes etotstar's numerator, and with it the last residual, NaN
 // or infinite.  No numerator is ever -0: each ends in a sum with +0 or with a number
 // that is not zero.
-template <bool FS = false, bool BND = false, class T>
+template <bool BND = false, class T>
 __device__ __forceinline__ void hllc(const SchemeT<T> &s, const Q4T<T> &ql, const Q4T<T> &qr,
                                      int ln, int tn, T flux[4], bool &ok) {
   using O = Ops<T>;
@@ -573,7 +572,7 @@ __device__ __forceinline__ void hllc(const SchemeT<T> &s, const Q4T<T> &ql, cons
   const T pr = O::mx(qr.v[IP], rr * s.smallp);
   const T ul = ql.v[ln], ur = qr.v[ln];
 
-  const T cmax = wave_speed<FS, BND>(s, pl, rl, pr, rr);
+  const T cmax = wave_speed<BND>(s, pl, rl, pr, rr);
   const T SL = O::mn(ul, ur) - cmax;
   const T SR = O::mx(ul, ur) + cmax;
 
@@ -644,7 +643,7 @@ __device__ __forceinline__ void hllc(const SchemeT<T> &s, const Q4T<T> &ql, cons
 // wave speeds of riemann_hllc.  Same expressions as the CPU oracle.  BND: SR - SL
 // is at least smallc wherever the middle state is taken, and below 2^313, so its
 // reciprocal needs no test.
-template <bool FS = false, bool BND = false, class T>
+template <bool BND = false, class T>
 __device__ __forceinline__ void hll(const SchemeT<T> &s, const Q4T<T> &ql, const Q4T<T> &qr,
                                     int ln, int tn, T flux[4]) {
   using O = Ops<T>;
@@ -656,7 +655,7 @@ __device__ __forceinline__ void hll(const SchemeT<T> &s, const Q4T<T> &ql, const
   const T ur = qr.v[ln], vr = qr.v[tn];
   const T el = O::mad(pl, s.entho, O::mad(h * rl * vl, vl, h * rl * ul * ul));
   const T er = O::mad(pr, s.entho, O::mad(h * rr * vr, vr, h * rr * ur * ur));
-  const T cmax = wave_speed<FS, BND>(s, pl, rl, pr, rr);
+  const T cmax = wave_speed<BND>(s, pl, rl, pr, rr);
   const T SL = O::mn(ul, ur) - cmax;
   const T SR = O::mx(ul, ur) + cmax;
   // variable order of the conserved state: rho, E, normal momentum, transverse momentum
@@ -765,9 +764,9 @@ __device__ __forceinline__ void approx(const SchemeT<T> &s, const Q4T<T> &qlf, c
 }
 
 // solver chosen at compile time: RS = 0 approx, 1 hll, 2 hllc
-// RS: 0 approx, 1 HLL, 2 HLLC; + kRiemannFloorSqrt: the HLL/HLLC wave speeds
-// use the short square root and, in the march, the bounded quotients (FP64,
-// where SchemeT::floor_sqrt holds)
+// RS: 0 approx, 1 HLL, 2 HLLC; + kRiemannFloorSqrt: the bounded quotients and the short
+// square root in the HLL / HLLC step and in its CFL rate (FP64, where
+// SchemeT::floor_sqrt holds)
 constexpr int kRiemannFloorSqrt = 8;
 // + kMinmodPow2: the march is built for slope_type == 1 (its slopes) and for
 // cell sizes that are powers of two (its CFL rate); the host selects such a
@@ -783,11 +782,10 @@ template <int RS, bool BND, class T>
 __device__ __forceinline__ void riemann(const SchemeT<T> &s, const Q4T<T> &ql, const Q4T<T> &qr,
                                         int ln, int tn, T flux[4], bool &ok) {
   constexpr int kind = RS & 7;
-  constexpr bool fs = (RS & kRiemannFloorSqrt) != 0;
   if constexpr (kind == 2)
-    hllc<fs, BND>(s, ql, qr, ln, tn, flux, ok);
+    hllc<BND>(s, ql, qr, ln, tn, flux, ok);
   else if constexpr (kind == 1)
-    hll<fs, BND>(s, ql, qr, ln, tn, flux);
+    hll<BND>(s, ql, qr, ln, tn, flux);
   else
     approx(s, ql, qr, ln, tn, flux);
 }
