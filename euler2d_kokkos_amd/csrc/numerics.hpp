@@ -527,9 +527,10 @@ __device__ __forceinline__ void trace_face(const SchemeT<T> &s, const Q4T<T> &q,
 // square root never decreases where its argument grows, so the root of the
 // larger argument is the larger root, bit for bit, and one root serves both
 // (the FP32 hardware root was checked to be monotone over every positive float).
-// BND: states in the bounded ranges, whose quotients and root take the short forms
-// (the short root would give NaN for the +inf that other states may bring).
-template <bool BND, class T>
+// FS: the short root, which would give NaN for the +inf that states outside the bounded
+// ranges may bring; the full root there costs every wavefront (768x384 16.9 -> 17.5 us a
+// step).  BND: quotients of states in the bounded ranges.
+template <bool FS, bool BND, class T>
 __device__ __forceinline__ T wave_speed(const SchemeT<T> &s, T pl, T rl, T pr, T rr) {
   using O = Ops<T>;
   if constexpr (BND) {
@@ -538,6 +539,7 @@ __device__ __forceinline__ T wave_speed(const SchemeT<T> &s, T pl, T rl, T pr, T
     return sqrt_core(O::mx(O::mx(xl, xr), s.smallc2));
   } else {
     const T a = O::mx(O::mx(O::div(s.gamma0 * pl, rl), O::div(s.gamma0 * pr, rr)), s.smallc2);
+    if constexpr (FS) return a > T(__DBL_MAX__) ? a : sqrt_core(a);
     return O::sqroot(a);
   }
 }
@@ -561,7 +563,7 @@ __device__ __forceinline__ T wave_speed(const SchemeT<T> &s, T pl, T rl, T pr, T
 // ustar or ptotstar makes etotstar's numerator, and with it the last residual, NaN
 // or infinite.  No numerator is ever -0: each ends in a sum with +0 or with a number
 // that is not zero.
-template <bool BND = false, class T>
+template <bool FS = false, bool BND = false, class T>
 __device__ __forceinline__ void hllc(const SchemeT<T> &s, const Q4T<T> &ql, const Q4T<T> &qr,
                                      int ln, int tn, T flux[4], bool &ok) {
   using O = Ops<T>;
@@ -572,7 +574,7 @@ __device__ __forceinline__ void hllc(const SchemeT<T> &s, const Q4T<T> &ql, cons
   const T pr = O::mx(qr.v[IP], rr * s.smallp);
   const T ul = ql.v[ln], ur = qr.v[ln];
 
-  const T cmax = wave_speed<BND>(s, pl, rl, pr, rr);
+  const T cmax = wave_speed<FS, BND>(s, pl, rl, pr, rr);
   const T SL = O::mn(ul, ur) - cmax;
   const T SR = O::mx(ul, ur) + cmax;
 
@@ -643,7 +645,7 @@ __device__ __forceinline__ void hllc(const SchemeT<T> &s, const Q4T<T> &ql, cons
 // wave speeds of riemann_hllc.  Same expressions as the CPU oracle.  BND: SR - SL
 // is at least smallc wherever the middle state is taken, and below 2^313, so its
 // reciprocal needs no test.
-template <bool BND = false, class T>
+template <bool FS = false, bool BND = false, class T>
 __device__ __forceinline__ void hll(const SchemeT<T> &s, const Q4T<T> &ql, const Q4T<T> &qr,
                                     int ln, int tn, T flux[4]) {
   using O = Ops<T>;
@@ -655,7 +657,7 @@ __device__ __forceinline__ void hll(const SchemeT<T> &s, const Q4T<T> &ql, const
   const T ur = qr.v[ln], vr = qr.v[tn];
   const T el = O::mad(pl, s.entho, O::mad(h * rl * vl, vl, h * rl * ul * ul));
   const T er = O::mad(pr, s.entho, O::mad(h * rr * vr, vr, h * rr * ur * ur));
-  const T cmax = wave_speed<BND>(s, pl, rl, pr, rr);
+  const T cmax = wave_speed<FS, BND>(s, pl, rl, pr, rr);
   const T SL = O::mn(ul, ur) - cmax;
   const T SR = O::mx(ul, ur) + cmax;
   // variable order of the conserved state: rho, E, normal momentum, transverse momentum
@@ -782,10 +784,11 @@ template <int RS, bool BND, class T>
 __device__ __forceinline__ void riemann(const SchemeT<T> &s, const Q4T<T> &ql, const Q4T<T> &qr,
                                         int ln, int tn, T flux[4], bool &ok) {
   constexpr int kind = RS & 7;
+  constexpr bool fs = (RS & kRiemannFloorSqrt) != 0;
   if constexpr (kind == 2)
-    hllc<BND>(s, ql, qr, ln, tn, flux, ok);
+    hllc<fs, BND>(s, ql, qr, ln, tn, flux, ok);
   else if constexpr (kind == 1)
-    hll<BND>(s, ql, qr, ln, tn, flux);
+    hll<fs, BND>(s, ql, qr, ln, tn, flux);
   else
     approx(s, ql, qr, ln, tn, flux);
 }
