@@ -1254,7 +1254,7 @@ __device__ __forceinline__ typename P::T march(const KParams &kp, const Grid &in
   m.rm1 = 0.0;
   m.rokm1 = false;
   m.ok1 = m.ok2 = true;
-  m.slow = !wave_all((double)dtdx <= kBndDtd && (double)dtdy <= kBndDtd);
+  m.slow = !wave_all(fabs(dt) <= kp.bnd_dt);
   m.wmax = T(0.0);
 
   const int r0 = j_base - 2;
@@ -1534,7 +1534,7 @@ void step_block_kernel(KParams kp, Grid in, Grid out, double dt_arg, StepCtl *ct
 #pragma unroll
   for (int k = 0; k < K; k++) {
     if constexpr (kBnd) {
-      bool rok, slow = !wave_all(dtdx <= kBndDtd && dtdy <= kBndDtd);
+      bool rok, slow = !wave_all(fabs(dt) <= kp.bnd_dt);
       const bool all = wave_all(P::template prim_shared<true>(kp, uc[k], q[k], rinv[k], rok));
       if (!all) {  // uniform
         P::prim_ieee(kp, uc[k], q[k]);
@@ -2212,6 +2212,7 @@ KParams make_kparams(const e2d_params &p, int precision) {
   k.nStepmax = p.nStepmax;
   k.dx = p.dx;
   k.dy = p.dy;
+  k.bnd_dt = kBndDtd * std::min(p.dx, p.dy);
   k.dxf = (float)p.dx;
   k.dyf = (float)p.dy;
   k.cfl = p.cfl;

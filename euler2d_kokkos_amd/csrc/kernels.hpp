@@ -33,6 +33,7 @@ struct KParams {
   int nStepmax;
   double dx, dy, cfl, tEnd;
   float dxf, dyf;
+  double bnd_dt;        // largest |dt| of the bounded FP64 forms (kBndDtd)
   RateT<double> rd;     // cell sizes of the CFL rate (FP64 / FP32 arithmetic)
   RateT<float> rf;
   // split path: primitive conversion redone in FP64 where the internal energy

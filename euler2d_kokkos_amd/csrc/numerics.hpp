@@ -121,7 +121,7 @@ using Q4 = Q4T<double>;
 // that their halves are exact (a zero residual alone would not bound them: over
 // d = 1 every denormal divides exactly).  E / d enters the pressure only;
 // p >= smallr smallp >= 2^-340 makes pressure differences zero or at least 2^-393.
-// With dt / dx <= 2^40 (checked per wavefront) the traced face states stay below
+// With |dt / dx| <= 2^40 (checked per wavefront) the traced face states stay below
 // 2^185 in density, 2^268 in pressure (2^455 once floored, for a large smallp) and
 // 2^311 in velocity, and the wave speeds below 2^200; what may still overflow in the
 // solvers is named there.  A wavefront with a lane outside these ranges takes the
@@ -151,7 +151,7 @@ constexpr int kClassNormal = (1 << 3) | (1 << 8);
 constexpr int kClassZeroOrNormal = kClassNormal | (1 << 5) | (1 << 6);
 
 constexpr double kBndDensity = 0x1p80, kBndPressure = 0x1p160, kBndKinetic = 0x1p120;
-constexpr double kBndDtd = 0x1p40;  // dt / dx, dt / dy
+constexpr double kBndDtd = 0x1p40;  // |dt / dx|, |dt / dy|
 constexpr int kBndMomentumExp = -800;  // frexp exponent: zero (exponent 0) or >= 2^-801
 
 // a / d from r = 1 / d where no step needs scaling and a is not -0
