@@ -208,8 +208,8 @@ int count_steps(e2d_run *r, long long upto) {
 }
 
 // One fused step with an explicit dt, queued with events of its own: the host
-// neither waits for the step nor makes events for it (together 30 us a call at
-// 512x512, more than the step).  The timers are brought up to date when they are
+// neither waits for the step nor makes events for it (together 27 of 47 us a call at
+// 512x512, twice the step).  The timers are brought up to date when they are
 // read, or when an event's slot comes round again.
 int queue_step(e2d_run *r, const Grid &in, const Grid &out, double dt) {
   int rc = count_steps(r, r->step_next - kStepEvents + 1);

@@ -1481,7 +1481,7 @@ void step_fused_kernel(KParams kp, Grid in, Grid out,
 // block runs per CU, so a step takes about 3 us of launch and loop control, one
 // memory round trip and the issue of the block's rows on four SIMDs (one row alone
 // 1.5 us, 20 rows 9 us).  Step time, the march at its best tile -> the block kernel:
-// FP64 64x64 8.3 -> 5.6 us, 256x256 10.9 -> 8.1, 501x363 15.3 -> 12.2, 512x512 17.5 -> 14.3.
+// FP64 64x64 8.3 -> 5.3 us, 256x256 10.9 -> 7.8, 501x363 15.3 -> 11.0, 512x512 15.9 -> 13.7.
 template <int RS, class P, int K, bool LOOP>
 __global__ __launch_bounds__(block_max_waves(K) * kLanes, block_max_waves(K) / 4)
 void step_block_kernel(KParams kp, Grid in, Grid out, double dt_arg, StepCtl *ctl, int ph) {
@@ -2387,8 +2387,8 @@ BlockMap block_map(const KParams &kp, int seg_rows) {
   m.nstrips = (kp.nx + kOutCols - 1) / kOutCols;
   m.nsegs = (kp.ny + rows - 1) / rows;
   // one block per CU: past that a second round of blocks costs a whole step again
-  // (512x512, 8 rows, 576 blocks: 19.8 us; 20 rows, 234 blocks: 14.1; the
-  // march's best 16.6)
+  // (512x512, 8 rows, 576 blocks: 19.8 us; 20 rows, 234 blocks: 13.7; the
+  // march's best 15.9)
   if ((long long)m.nstrips * m.nsegs <= kp.simds / 4) m.k = k;
   return m;
 }

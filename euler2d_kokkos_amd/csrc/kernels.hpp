@@ -171,19 +171,19 @@ BlockMap block_map(const KParams &kp, int seg_rows);
 // warm-up rows worth two) on `simds` SIMDs that hold two at a time: two that
 // share a SIMD take 2 units a row, one alone 1.35.  Against measured times: FP64
 // 1024x1536, tiles 7 / 10 / 12 / 14 / 16 / 20: 36 / 38 / 47 / 32 / 36 / 44 units,
-// 51.0 / 52.8 / 59.2 / 43.6 / 49.5 / 55.8 us; 3001x1777, tiles 14 / 24 / 48: 118 / 104 / 100
-// units, 160 / 154 / 144 us.
+// 50.9 / 52.9 / 59.4 / 43.9 / 49.4 / 55.8 us; 3001x1777, tiles 14 / 24 / 48: 118 / 104 / 100
+// units, 141 / 137 / 125 us.
 double march_cost(double waves, int tile, int simds);
 // Split precision over more than eight rounds of wavefronts (counted at kSplitTile rows)
 // is bound by memory: short segments keep more of the halo rows in the caches than the
-// cost's longer ones.  8192x8192, 14 / 60 rows: 1022 / 1078 us a step; 16384x8192 2011 /
-// 2062; 4096x4096 266 / 271; 192 grids of 64 .. 512 219 / 235.  At six rounds (3001x1777)
-// the cost's tile wins: 85.8 against 90.7.
+// cost's longer ones.  8192x8192, 14 / 60 rows: 970 / 1011 us a step; 16384x8192 1867 /
+// 1934; 4096x4096 258 / 270; 192 grids of 64 .. 512 219 / 235.  At six rounds (3001x1777)
+// the cost's tile wins: 83.5 against 89.2.
 constexpr int kSplitTile = 14;
 bool many_rounds_split(const KParams &kp, double waves);
 // The tile a run starts with: the smallest whose blocks fit one per CU (a
 // smaller one shortens each wavefront's chain as long as no second round of
-// blocks is needed: 256x256, tiles 6 / 8 / 12: 8.1 / 8.5 / 10.1 us); for larger
+// blocks is needed: 256x256, tiles 6 / 8 / 12: 7.7 / 8.3 / 9.8 us); for larger
 // grids the march's tile of least march_cost.
 int auto_tile(const KParams &kp);
 
